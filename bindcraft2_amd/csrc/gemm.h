@@ -29,10 +29,6 @@ namespace bc2n {
 
 struct GemmArgs {
   int M = 0, N = 0, K = 0, batch = 1;
-  // > 0 (the sliced launch): the accumulators fold into the result every
-  // kslice of K, in order, giving the bits of a split-K launch of kslice
-  // slices summed by gemm_splitk_epi, on a grid of the tiles alone
-  int kslice = 0;
   const h16* A = nullptr;
   long a_sm = 0, a_sk = 0, a_sb = 0;  // element strides; a_sm==1 or a_sk==1
   const h16* B = nullptr;
@@ -202,11 +198,9 @@ template <class E>
 struct epi_min_waves<E, std::void_t<decltype(E::kMinWaves)>>
     : std::integral_constant<int, E::kMinWaves> {};
 
-template <int BM, int BN, int BK, bool AK, bool BKC, class Epi, class AL = ALoadDirect,
-          bool SLICED = false>
+template <int BM, int BN, int BK, bool AK, bool BKC, class Epi, class AL = ALoadDirect>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(epi_min_waves<Epi>::value)))
 void gemm_kernel(GemmArgs g, Epi epi, AL al = AL{}) {
-  static_assert(!SLICED || BK == 32, "the sliced launch folds at 32-deep steps");
   using SM = GemmSmem<BM, BN, BK>;
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
@@ -317,7 +311,6 @@ void gemm_kernel(GemmArgs g, Epi epi, AL al = AL{}) {
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int nk = g.K / BK;
-  f32x4 total[SLICED ? TM : 1][SLICED ? TN : 1];  // the slices' running sum
   constexpr int PRO = epi_pro_floats<Epi>::value;
   __shared__ float pro[PRO > 0 ? BM * PRO : 1];
   gload(0);
@@ -350,21 +343,6 @@ void gemm_kernel(GemmArgs g, Epi epi, AL al = AL{}) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x32(af[i], bfr[j], acc[i][j]);
     }
-    if constexpr (SLICED) {
-      // a slice ends: its partial joins the running sum (the first one as
-      // it is, as gemm_splitk_epi starts from partial 0) and restarts at 0
-      const int spk = g.kslice / 32;
-      if ((kt + 1) % spk == 0) {
-        const bool first = kt + 1 == spk;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            total[i][j] = first ? acc[i][j] : total[i][j] + acc[i][j];
-            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
-      }
-    }
     if constexpr (SM::NBUF == 2) {
       if (kt + 1 < nk) sstore(buf ^ 1);
     } else if (kt + 1 < nk) {
@@ -372,13 +350,6 @@ void gemm_kernel(GemmArgs g, Epi epi, AL al = AL{}) {
       sstore(0);
     }
     __syncthreads();
-  }
-
-  if constexpr (SLICED) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j];
   }
 
   // ---- epilogue: stage half a tile (the rows of one wave row) per pass
@@ -472,20 +443,156 @@ void gemm_launch(hipStream_t st, const GemmArgs& g, const Epi& epi, const AL& al
 #undef BC2N_GEMM_LAUNCH
 }
 
-// The sliced launch (g.kslice > 0, a multiple of 32 dividing K): 32-deep
-// steps, a grid of the tiles alone.
-template <int BM, int BN, class Epi, class AL>
-void gemm_launch_sliced(hipStream_t st, const GemmArgs& g, const Epi& epi, const AL& al) {
-  const bool ak = (g.a_sk == 1), bk = (g.b_sk == 1);
-  const int tiles = ((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
-  dim3 grid(xcd_grid((long)tiles * g.batch)), block(256);
-#define BC2N_GEMM_SLICED(AKV, BKCV) \
-  hipLaunchKernelGGL((gemm_kernel<BM, BN, 32, AKV, BKCV, Epi, AL, true>), grid, block, 0, st, g, epi, al)
-  if (ak && bk) BC2N_GEMM_SLICED(true, true);
-  else if (ak) BC2N_GEMM_SLICED(true, false);
-  else if (bk) BC2N_GEMM_SLICED(false, true);
-  else BC2N_GEMM_SLICED(false, false);
-#undef BC2N_GEMM_SLICED
+// Products of a few tiles (the MSA's S x N rows: 160 x 256 over K = 1024 is
+// four tiles of 128 x 128): with an LDS-staged tile they are one or two waves'
+// chain of dependent K steps on a handful of CUs, bound by load latency (26 to
+// 34 us a launch).  Here a workgroup owns a tile of 16 or 32 rows, its waves
+// read their fragments straight from memory (no LDS staging, up to U 32-deep
+// steps in flight, so a wave waits about once), and the K slices of a split
+// product run on different waves instead of different workgroups:
+//
+//  WS = 4: wave w takes slices w, w + 4, ... of the whole tile; every slice's
+//          partial goes to LDS and the epilogue adds them in slice order
+//  WS = 1: the four waves take the tile's column quarters, each folding its
+//          slices in order (fewer than four slices)
+//
+// Either way a result is the slices' 32-deep MFMA chains added in slice order:
+// the bits of a split launch summed by gemm_splitk_epi, without its partials
+// in memory and its second launch.
+template <int TM, int TN, int WS, int U, class Epi, class AL>
+__global__ __launch_bounds__(256) void gemm_few_kernel(GemmArgs g, int split, Epi epi, AL al) {
+  constexpr int WN = 4 / WS;                        // column groups
+  constexpr int BM = 16 * TM, BN = 16 * TN * WN, LDP = BN + 4;
+  extern __shared__ __attribute__((aligned(16))) float few_part[];  // [slices or 1][BM][LDP]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ws = wave % WS, wn = wave / WS;
+  const int tiles_n = (g.N + BN - 1) / BN;
+  const long tiles = (long)((g.M + BM - 1) / BM) * tiles_n;
+  const long t = xcd_block(tiles);
+  if (t >= tiles) return;
+  const int m0 = (int)(t / tiles_n) * BM, n0 = (int)(t % tiles_n) * BN;
+  const int fr = lane & 15, fk = (lane >> 4) * 8;
+
+  // rows past M (columns past N) read the last one and store nothing
+  int am[TM];
+  const h16* bp[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) am[i] = min(m0 + i * 16 + fr, g.M - 1);
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+    bp[j] = g.B + (long)min(n0 + (wn * TN + j) * 16 + fr, g.N - 1) * g.b_sn + fk;
+
+  const int spk = g.K / 32 / split;                  // 32-deep steps a slice
+  const int nst = (split - ws + WS - 1) / WS * spk;   // this wave's steps (split >= WS)
+  f32x4 acc[TM][TN], total[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto put = [&](const f32x4 (&a)[TM][TN], int slot) __attribute__((always_inline)) {
+    float* P = few_part + (long)slot * BM * LDP;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          P[(i * 16 + (lane >> 4) * 4 + r) * LDP + (wn * TN + j) * 16 + fr] = a[i][j][r];
+  };
+
+  int ls = ws, lk = 0;  // the next step to load: slice, step in it
+  int cs = ws, ck = 0;  // the next step to compute
+  for (int base = 0; base < nst; base += U) {
+    h16x8 af[U][TM], bf[U][TN];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (base + u >= nst) break;  // wave-uniform
+      const int k = (ls * spk + lk) * 32;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        if constexpr (AL::kDirect) af[u][i] = ld8(g.A + (long)am[i] * g.a_sm + k + fk);
+        else af[u][i] = al(0, am[i], k + fk);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bf[u][j] = ld8(bp[j] + k);
+      if (++lk == spk) {
+        lk = 0;
+        ls += WS;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (base + u >= nst) break;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x32(af[u][i], bf[u][j], acc[i][j]);
+      if (++ck == spk) {  // the slice is done
+        if constexpr (WS > 1) {
+          put(acc, cs);
+        } else {
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) total[i][j] = cs == 0 ? acc[i][j] : total[i][j] + acc[i][j];
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        ck = 0;
+        cs += WS;
+      }
+    }
+  }
+  if constexpr (WS == 1) put(total, 0);
+  __syncthreads();
+  const int slots = WS > 1 ? split : 1;
+  for (int it = tid; it < BM * (BN / 8); it += 256) {
+    const int r = it / (BN / 8), c8 = (it % (BN / 8)) * 8;
+    const int m = m0 + r, n = n0 + c8;
+    if (m >= g.M || n >= g.N) continue;
+    const float* P = few_part + r * LDP + c8;
+    float v[8];
+    ld_f8(P, v);
+    for (int s = 1; s < slots; ++s) {
+      float w[8];
+      ld_f8(P + (long)s * BM * LDP, w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += w[e];
+    }
+    epi.row(0, m, n, v);
+  }
+}
+
+// Slices at most (their partials share a workgroup's LDS: 36 KB for 16).
+constexpr int GEMM_FEW_MAX_SLICES = 16;
+
+// Both operands K-contiguous, one batch entry, `split` slices of a multiple
+// of 32.  16-row tiles while they leave CUs to fill; the 32 x 64 tile, which
+// reads half the operand bytes a product, once 16 x 32 tiles exceed four a CU
+// (only for up to four slices: its partials take 9 KB each).
+template <class Epi, class AL>
+void gemm_few(hipStream_t st, const GemmArgs& g, int split, const Epi& epi, const AL& al) {
+  const long t32 = (long)((g.M + 15) / 16) * ((g.N + 31) / 32);
+  auto go = [&](auto tm, auto tn, auto ws, auto u) {
+    constexpr int TM = decltype(tm)::value, TN = decltype(tn)::value, WS = decltype(ws)::value;
+    constexpr int BM = 16 * TM, BN = 16 * TN * (4 / WS);
+    const long tiles = (long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    const size_t lds = (size_t)(WS > 1 ? split : 1) * BM * (BN + 4) * 4;
+    hipLaunchKernelGGL((gemm_few_kernel<TM, TN, WS, decltype(u)::value, Epi, AL>),
+                       dim3(xcd_grid(tiles)), dim3(256), lds, st, g, split, epi, al);
+  };
+  using std::integral_constant;
+  const integral_constant<int, 1> c1{};
+  const integral_constant<int, 2> c2{};
+  const integral_constant<int, 4> c4{};
+  const integral_constant<int, 8> c8{};
+  if (split < 4) go(c1, c1, c1, c8);
+  else if (split == 4 && t32 > 4L * device_cus()) go(c2, c4, c4, c2);
+  else if (g.K / 32 / split * ((split + 3) / 4) <= 2) go(c1, c2, c4, c2);
+  else go(c1, c2, c4, c8);
 }
 
 // Split K for a grid of a few tiles and a long K (the MSA track's S x N-row
@@ -571,24 +678,20 @@ void gemm(hipStream_t st, const GemmArgs& g, const Epi& epi, const char* name = 
   KTimed kt(name, st);
   constexpr bool kSplittable = !epi_row_block<Epi>::value && !Epi::kHasCol && !AL::kSide;
   if constexpr (kSplittable) {
-    if (g.batch == 1 && tiles * 2 < device_cus() && g.K >= 256 && g.N % 64 == 0) {
+    if (g.batch == 1 && tiles * 2 < device_cus()) {
       // slices of at least 64 (a multiple of 32 that divides K), about one
-      // workgroup per CU in all
-      const int kb = g.K / 32;
-      int split = (int)std::min<long>((device_cus() + tiles - 1) / tiles, g.K / 64);
-      while (split > 1 && kb % split != 0) --split;
+      // 128-row workgroup per CU in all
+      int split = 1;
+      if (g.K >= 256 && g.N % 64 == 0) {
+        split = (int)std::min<long>((device_cus() + tiles - 1) / tiles, g.K / 64);
+        while (split > 1 && g.K / 32 % split != 0) --split;
+      }
+      if (ak && bk && split <= GEMM_FEW_MAX_SLICES) {
+        gemm_few(st, g, split, epi, al);
+        return;
+      }
       if (split > 1) {
         const int kslice = g.K / split;
-        if (lane() != 0) {
-          // the side lane runs beside the pair track, the critical path: the
-          // same sums on a grid of the tiles alone (no extra workgroups, no
-          // partials through memory, no reduction launch) take less of the
-          // chip from it; the bits are those of the split launch
-          GemmArgs gk = g;
-          gk.kslice = kslice;
-          gemm_launch_sliced<BM, BN>(st, gk, epi, al);
-          return;
-        }
         GemmArgs gs = g;
         gs.K = kslice;
         gs.batch = split;
