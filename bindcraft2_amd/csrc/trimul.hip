@@ -277,7 +277,7 @@ struct EpiCmLnBwd : EpiRows {
 };
 
 // ---------------------------------------------------------------------------
-// The backward's tail in one kernel (C = I = 128):
+// The backward's tail in one kernel (I = C, C = 128 or 64):
 //
 //   P   = xn . Wcat[:, :4I]                    (recompute, K = C)
 //   d(cat)[:, :4I] from P, d(left|right), mask (the EpiTrimulProjBwd formulas)
@@ -285,280 +285,313 @@ struct EpiCmLnBwd : EpiRows {
 //                                               of d(cat) come from memory)
 //   din = dout + LN'(dy)                       (the input LayerNorm's backward)
 //
-// d(cat)'s [proj|gate] columns never leave registers: GEMM1 runs transposed
-// (the weights as the first MFMA operand), so a lane ends with row m = l%16 and
-// 4 consecutive columns 4g..4g+3 of a 16-column block.  The proj block and its
-// gate block (16 columns to the right) land in the same lane positions, so the
-// epilogue pairs them in registers, and the 8 values {proj 4g..4g+3, gate
-// 4g..4g+3} of a 32-column block are exactly one k-slot set of a 32-deep MFMA
-// step of GEMM2 -- the same slot order that its weights are read in.  GEMM2
-// also runs transposed, so each lane holds 32 channels (16j + 4g + r) of its
-// row for the LayerNorm's row sums (completed across the 4 lanes of the row).
+// A workgroup owns 16 RT rows: its xn tile (k order permuted inside 32-blocks,
+// below) and its d(left|right) tile (channel-major, as in memory) are in LDS
+// before the first product, so the chunk loop waits on memory for weight
+// fragments alone, and those are loaded a chunk ahead.  The [proj|gate]
+// columns are made and consumed 128 at a time.  The four waves split the
+// columns of both products over all rows (every weight fragment is read once
+// a workgroup, straight from memory, one contiguous 1 KB a wave):
 //
-// Workgroup: 128 rows, 4 waves of 32 rows (two 16-row tiles).  The weights
-// stream through LDS in 10 chunks (8 of 64 GEMM1 columns, with the matching
-// 64 rows of GEMM2's K, and 2 chunks of the gating_linear K), double-buffered
-// with a register prefetch of the next chunk.
-namespace tail {
-constexpr int C = 128, I = 128, NC = 4 * I + C;
-constexpr int RT = 2;                     // 16-row tiles per wave
-constexpr int BM = 64 * RT;               // rows per workgroup (4 waves)
-constexpr int CH = 64;                    // GEMM1 columns (= GEMM2 k) per chunk
-constexpr int NPG = 4 * I / CH;           // [proj|gate] chunks
-constexpr int NCHUNK = NPG + C / CH;      // + gating_linear chunks
-// row strides = 8 (mod 64) dwords: the 16-byte fragment reads of 16 rows are
-// bank-conflict free
-constexpr int LD1 = C + 16;               // B1 chunk: [CH][C] (n rows, k contiguous)
-constexpr int LD2 = CH + 16;              // B2 chunk: [C][CH] (c rows, k contiguous)
-constexpr int B1E = CH * LD1, B2E = C * LD2;
-}  // namespace tail
-
-// 8 h16 of row `row` at k = k0 + {4g..4g+3, 16+4g..16+4g+3} of a
-// K-contiguous tile (row stride ld), global or LDS.
-__device__ __forceinline__ h16x8 kslots(const h16* T, long ld, long row, int k0, int g) {
-  const h16* p = T + row * ld + k0 + 4 * g;
-  const h16x4 a = *reinterpret_cast<const h16x4*>(p);
-  const h16x4 b = *reinterpret_cast<const h16x4*>(p + 16);
-  h16x8 r;
-  r[0] = a[0]; r[1] = a[1]; r[2] = a[2]; r[3] = a[3];
-  r[4] = b[0]; r[5] = b[1]; r[6] = b[2]; r[7] = b[3];
-  return r;
-}
-
-// The weights' k order in the tail kernel's copies: within each 32-block,
-// physical position 8g + e holds logical k = 4g + e (e < 4) and 8g + 4 + e
-// holds 16 + 4g + e, so kslots' 8 values are 16 contiguous bytes.
-inline int tail_kperm(int p) {
-  const int b = p & ~31, g = (p & 31) >> 3, e = p & 7;
-  return b + (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4);
-}
+//  GEMM1, transposed (the weights as the first MFMA operand): wave w makes
+//    the chunk's 32-column block w, 16 proj columns and their 16 gates, and
+//    ends with row l%16 and columns 4g..4g+3 of both, so d(cat) is formed in
+//    registers, with d(left|right) from one transposed LDS read (channels
+//    4g..4g+3 of row l%16).  The 8 values {proj 4g..4g+3, gate 4g..4g+3} are
+//    one k-slot set of a 32-deep MFMA step: one 16-byte LDS store, one
+//    16-byte read as GEMM2's operand.
+//  GEMM2, transposed: wave w accumulates C / 4 output channels.
+//
+// Both products' K order and the row sums' order are those of the kernel this
+// one replaced (128 rows a workgroup, the waves splitting rows, the weights
+// streamed through LDS in ten barriers), whose bits it keeps.  That one was a
+// chain of ten exposed prefetches in too few workgroups: 32 us at N = 128
+// (128 workgroups) and 45 us at N = 224.
+template <int C_, int RT_>
+struct Tail {
+  static constexpr int C = C_, I = C_, NC = 4 * I + C, RT = RT_, BM = 16 * RT;
+  static constexpr int KS = C / 32;         // GEMM1's 32-deep steps
+  static constexpr int NPG = 4 * I / 128;   // chunks of [proj|gate] columns
+  static constexpr int JJ = C / 64;         // 16-channel output tiles a wave
+  static constexpr int LDX = C + 8, LDH = 128 + 8, LDT = C + 4;
+  static constexpr int LDD = BM % 32 == 16 ? BM : BM + 16;  // 16 mod 32: transposed reads
+  static constexpr int XS = BM * LDX * 2, HS = BM * LDH * 2, T = BM * LDT * 4;
+  static constexpr int MAIN = XS + HS > T ? XS + HS : T;  // xs, hs; the f32 output tile over both
+  static constexpr int DS = 2 * I * LDD * 2;
+};
 
 struct TailArgs {
-  const h16* xn;      // [M][C]
-  const h16* wcat_t;  // [NC][C], k permuted (tail_kperm)
-  const h16* wcat;    // [C][NC], k permuted (tail_kperm)
-  const h16 *dl, *dr; // [I][M]
-  const h16* dcg;     // [M][C]: d(cat)'s gating_linear columns
+  const h16* xn;       // [M][C]
+  const h16 *w1, *w2;  // tail_frags1 / tail_frags2
+  const h16 *dl, *dr;  // [I][M]
+  const h16* dcg;      // [M][C]: d(cat)'s gating_linear columns
   const float *bp, *bg, *mask;
   const float *x, *ln_g, *mean, *rstd, *dres;
-  const float* gmul;  // inverse cotangent scale (device scalar)
+  const float* gmul;   // inverse cotangent scale (device scalar)
   float* out;
   long M;
 };
 
-__global__ __launch_bounds__(256, 2) void trimul_tail_kernel(TailArgs a) {
-  using namespace tail;
-  __shared__ __attribute__((aligned(16))) h16 B1s[2 * B1E];
-  __shared__ __attribute__((aligned(16))) h16 B2s[2 * B2E];
-  // the projection biases, read in the d(cat) formulas from LDS: a global
-  // load there would wait (in-order vmcnt) for the next chunk's prefetch
-  __shared__ __attribute__((aligned(16))) float Bps[2 * I], Bgs[2 * I];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, l16 = lane & 15;
-  const long m0 = (long)blockIdx.x * BM + wave * 16 * RT;
-  const long M = a.M;
+// The k order of the LDS tiles and weight fragments: inside a 32-block lane
+// group g's 8 values are k = {4g..4g+3, 16+4g..16+4g+3}.
+__host__ __device__ inline int tail_k(int g, int e) { return e < 4 ? 4 * g + e : 12 + 4 * g + e; }
 
-  // ---- chunk staging: 16 KB of B1 and 16 KB of B2 per chunk, 4 + 4 16-byte pieces a thread
-  // Chunk s's operands are fetched during chunk s - 1: its weights into
-  // p1/p2 (stored to LDS at the end of chunk s - 1), and the lane's own
-  // operands into registers -- d(left|right) at its rows and channels (da) for
-  // a [proj|gate] chunk, its d(cat) gating fragments (in p1) for the others.
-  // The weights are issued first, so waiting for them leaves the rest in flight.
-  h16x8 p1[4], p2[4];
-  h16 da[RT][2][4];
-  auto prefetch = [&](int s) {
-    if (s < NPG) {
+// 8 consecutive k (k8 % 8 == 0) of one row into its permuted 32-block.
+__device__ __forceinline__ void tail_put(h16* row, int k8, h16x8 v) {
+  const int q = (k8 >> 3) & 3;
+  h16* p = row + (k8 & ~31) + 16 * (q & 1) + 4 * (q >> 1);
+  *reinterpret_cast<h16x4*>(p) = h16x4{v[0], v[1], v[2], v[3]};
+  *reinterpret_cast<h16x4*>(p + 8) = h16x4{v[4], v[5], v[6], v[7]};
+}
+
+template <int C_, int RT_>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void trimul_tail_kernel(
+    TailArgs a) {
+  using K = Tail<C_, RT_>;
+  constexpr int C = K::C, I = K::I, RT = K::RT, BM = K::BM, JJ = K::JJ, KS = K::KS;
+  __shared__ __attribute__((aligned(16))) char smem[K::MAIN];
+  __shared__ __attribute__((aligned(16))) h16 ds[2 * I * K::LDD];
+  __shared__ __attribute__((aligned(16))) float bps[2 * I], bgs[2 * I];
+  h16* xs = reinterpret_cast<h16*>(smem);
+  h16* hs = reinterpret_cast<h16*>(smem + K::XS);
+  float* T = reinterpret_cast<float*>(smem);
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long M = a.M, nwg = (M + BM - 1) / BM;
+  // neighbours share lines of d(left|right)'s planes: one XCD a range of rows
+  const long blk = xcd_block(nwg);
+  if (blk >= nwg) return;
+  const long m0 = blk * BM;
+
+  h16x8 b1[KS][2], b2[4][JJ];
+  auto load_b1 = [&](int j) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int c = tid + 256 * q, r = c / (C / 8), k8 = (c % (C / 8)) * 8;
-        p1[q] = ld8(a.wcat_t + (long)(s * CH + r) * C + k8);
-      }
-    }
-    const int kb = s < NPG ? s * CH : 4 * I + (s - NPG) * CH;
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c = tid + 256 * q, r = c / (CH / 8), k8 = (c % (CH / 8)) * 8;
-      p2[q] = ld8(a.wcat + (long)r * NC + kb + k8);
-    }
-    if (s < NPG) {
-      const h16* dsrc = s < NPG / 2 ? a.dl : a.dr;
-      const int chb = (s % (NPG / 2)) * 32;  // channel within left or right
+      for (int q = 0; q < 2; ++q)
+        b1[ks][q] = ld8(a.w1 + ((long)(((j * 4 + w) * 2 + q) * KS + ks) * 64 + lane) * 8);
+  };
+  auto load_b2 = [&](int j, int nb) {
 #pragma unroll
-      for (int i = 0; i < RT; ++i)
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+      for (int jj = 0; jj < JJ; ++jj)
+        if (b < nb) b2[b][jj] = ld8(a.w2 + ((long)(((j * 4 + b) * 4 + w) * JJ + jj) * 64 + lane) * 8);
+  };
+  // a [BM][C] tile, 16 bytes a piece; rows past M read row M - 1 (their
+  // results are never stored)
+  constexpr int XP = (BM * C / 8 + 255) / 256;
+  auto load_rows = [&](const h16* src, h16x8 (&v)[XP]) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            da[i][q][r] = dsrc[(long)(chb + q * 16 + 4 * g + r) * M + m0 + i * 16 + l16];
-    } else {
-      const int kc = (s - NPG) * CH;
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) p1[2 * i + q] = kslots(a.dcg, C, m0 + i * 16 + l16, kc + q * 32, g);
+    for (int p = 0; p < XP; ++p) {
+      const int it = min(tid + 256 * p, BM * C / 8 - 1);
+      v[p] = ld8(src + min(m0 + it / (C / 8), M - 1) * C + (it % (C / 8)) * 8);
     }
   };
-  auto stash = [&](int s, int buf) {
-    if (s < NPG) {
+  auto put_rows = [&](const h16x8 (&v)[XP]) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int c = tid + 256 * q, r = c / (C / 8), k8 = (c % (C / 8)) * 8;
-        st8(B1s + buf * B1E + r * LD1 + k8, p1[q]);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c = tid + 256 * q, r = c / (CH / 8), k8 = (c % (CH / 8)) * 8;
-      st8(B2s + buf * B2E + r * LD2 + k8, p2[q]);
+    for (int p = 0; p < XP; ++p) {
+      const int it = tid + 256 * p;
+      if (it < BM * C / 8) tail_put(xs + it / (C / 8) * K::LDX, (it % (C / 8)) * 8, v[p]);
     }
   };
 
-  prefetch(0);
-  // xn fragments of the wave's two row tiles, all of K, in GEMM1's slot order
-  h16x8 xf[RT][C / 32];
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int ks = 0; ks < C / 32; ++ks) xf[i][ks] = kslots(a.xn, C, m0 + i * 16 + l16, ks * 32, g);
+  // front: every load of both tiles before the first store
   float mk[RT];
+  h16x8 xv[XP];
+  {
+    constexpr int DP = (2 * I * (BM / 8) + 255) / 256;
+    h16x8 dv[DP];
+    load_rows(a.xn, xv);
 #pragma unroll
-  for (int i = 0; i < RT; ++i) mk[i] = a.mask[m0 + i * 16 + l16];
-  if (tid < 2 * I) {
-    Bps[tid] = a.bp[tid];
-    Bgs[tid] = a.bg[tid];
+    for (int p = 0; p < DP; ++p) {
+      const int it = min(tid + 256 * p, 2 * I * (BM / 8) - 1), ch = it / (BM / 8);
+      const h16* plane = ch < I ? a.dl + (long)ch * M : a.dr + (long)(ch - I) * M;
+      dv[p] = ld8(plane + min(m0 + (it % (BM / 8)) * 8, M - 8));
+    }
+    float bpv = 0.f, bgv = 0.f;
+    if (tid < 2 * I) {
+      bpv = a.bp[tid];
+      bgv = a.bg[tid];
+    }
+#pragma unroll
+    for (int i = 0; i < RT; ++i) mk[i] = a.mask[min(m0 + i * 16 + l16, M - 1)];
+    load_b1(0);
+    load_b2(0, 4);
+    put_rows(xv);
+#pragma unroll
+    for (int p = 0; p < DP; ++p) {
+      const int it = tid + 256 * p;
+      if (it < 2 * I * (BM / 8)) st8(ds + it / (BM / 8) * K::LDD + (it % (BM / 8)) * 8, dv[p]);
+    }
+    if (tid < 2 * I) {
+      bps[tid] = bpv;
+      bgs[tid] = bgv;
+    }
   }
-  stash(0, 0);
   __syncthreads();
 
-  float4 xpre[RT][C / 16];
-  f32x4 acc2[RT][C / 16];
+  f32x4 acc2[RT][JJ];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < C / 16; ++j) acc2[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < JJ; ++jj) acc2[i][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // fully unrolled: every chunk's registers are fixed at compile time, so the
-  // prefetched operands stay in flight until their use (no loop-carried copies)
 #pragma unroll
-  for (int s = 0; s < NCHUNK; ++s) {
-    const int buf = s & 1;
-    const h16* b1 = B1s + buf * B1E;
-    const h16* b2 = B2s + buf * B2E;
-    h16x8 af[RT][2];  // GEMM2 A fragments: [row tile][k-step of this chunk]
-    if (s < NPG) {
-      // GEMM1: P for 4 column blocks (proj, gate, proj, gate)
-      f32x4 acc1[RT][4];
+  for (int j = 0; j < K::NPG; ++j) {
+    // GEMM1: proj and gate columns of channels 16 (4j + w) + 4g + r, row i*16 + l16
+    f32x4 acc1[RT][2];
 #pragma unroll
-      for (int i = 0; i < RT; ++i)
+    for (int i = 0; i < RT; ++i) acc1[i][0] = acc1[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc1[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int ks = 0; ks < C / 32; ++ks) {
-        h16x8 bfr[4];
+      for (int i = 0; i < RT; ++i) {
+        const h16x8 xf = ld8(xs + (i * 16 + l16) * K::LDX + ks * 32 + 8 * g);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) bfr[t] = ld8(b1 + (t * 16 + l16) * LD1 + ks * 32 + 8 * g);
-#pragma unroll
-        for (int i = 0; i < RT; ++i)
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            acc1[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bfr[t], xf[i][ks], acc1[i][t], 0, 0, 0);
+        for (int q = 0; q < 2; ++q) acc1[i][q] = mfma16x16x32(b1[ks][q], xf, acc1[i][q]);
       }
-      // epilogue: d(proj) = a * sigmoid(gate), d(gate) = a * proj * s (1 - s), a = d(act) * mask
+    if (j + 1 < K::NPG) load_b1(j + 1);
+    else load_rows(a.dcg, xv);  // the gating_linear columns take xs next
+    // d(proj) = a * sigmoid(gate), d(gate) = a * proj * s (1 - s), a = d(act) * mask
+    const int ch = 16 * (4 * j + w) + 4 * g;
+    const float4 p4 = *reinterpret_cast<const float4*>(bps + ch);
+    const float4 g4 = *reinterpret_cast<const float4*>(bgs + ch);
+    const float bpv[4] = {p4.x, p4.y, p4.z, p4.w}, bgv[4] = {g4.x, g4.y, g4.z, g4.w};
+    h16x8 f[RT];
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int ch = s * 32 + q * 16 + 4 * g;  // channel of slot r = ch + r (0..2I)
-        float bpv[4], bgv[4];
+    for (int i = 0; i < RT; ++i) {
+      const h16x4 da = gemm_tr4(ds, K::LDD, 16 * (4 * j + w), i * 16, lane);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) { bpv[r] = Bps[ch + r]; bgv[r] = Bgs[ch + r]; }
-#pragma unroll
-        for (int i = 0; i < RT; ++i) {
-          h16x8 f;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float pv = acc1[i][2 * q][r] + bpv[r];
-            const float sg = sigmoidf_(acc1[i][2 * q + 1][r] + bgv[r]);
-            const float ad = (float)da[i][q][r] * mk[i];
-            f[r] = f2h_sat(ad * sg);
-            f[4 + r] = f2h_sat(ad * pv * sg * (1.f - sg));
-          }
-          af[i][q] = f;
-        }
-      }
-    } else {
-      // gating_linear columns of d(cat), fetched during the previous chunk
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) af[i][q] = p1[2 * i + q];
-    }
-    // the next chunk's operands load behind GEMM2 (the weights are
-    // L2-resident: every workgroup reads the same 288 KB)
-    if (s + 1 < NCHUNK) prefetch(s + 1);
-    if (s == NPG) {
-      // the LayerNorm tail's x rows, loaded behind the last two chunks (GEMM1
-      // is done, so its operand registers are free)
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int j = 0; j < C / 16; ++j)
-          xpre[i][j] = *reinterpret_cast<const float4*>(a.x + (m0 + i * 16 + l16) * C + 16 * j + 4 * g);
-    }
-    // GEMM2: dy[m][c] += d(cat)[m][k] Wcat[c][k] over the chunk's 64 k
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-#pragma unroll
-      for (int j = 0; j < C / 16; ++j) {
-        const h16x8 bfr = ld8(b2 + (j * 16 + l16) * LD2 + q * 32 + 8 * g);
-#pragma unroll
-        for (int i = 0; i < RT; ++i)
-          acc2[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bfr, af[i][q], acc2[i][j], 0, 0, 0);
+      for (int r = 0; r < 4; ++r) {
+        const float pv = acc1[i][0][r] + bpv[r];
+        const float sg = sigmoidf_(acc1[i][1][r] + bgv[r]);
+        const float ad = (float)da[r] * mk[i];
+        f[i][r] = f2h_sat(ad * sg);
+        f[i][4 + r] = f2h_sat(ad * pv * sg * (1.f - sg));
       }
     }
-    if (s + 1 < NCHUNK) stash(s + 1, buf ^ 1);
+    if (j > 0) __syncthreads();  // the previous chunk's GEMM2 is done with hs
+#pragma unroll
+    for (int i = 0; i < RT; ++i) st8(hs + (i * 16 + l16) * K::LDH + 32 * w + 8 * g, f[i]);
     __syncthreads();
+    if (j == K::NPG - 1) put_rows(xv);  // every wave is past its last read of xn
+    // GEMM2: output channels 16 (JJ w + jj) + 4g + r of row i*16 + l16
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const h16x8 af = ld8(hs + (i * 16 + l16) * K::LDH + b * 32 + 8 * g);
+#pragma unroll
+        for (int jj = 0; jj < JJ; ++jj) acc2[i][jj] = mfma16x16x32(b2[b][jj], af, acc2[i][jj]);
+      }
+    load_b2(j + 1, j + 1 < K::NPG ? 4 : KS);
   }
+  __syncthreads();  // the gating_linear columns are in xs
 
-  // ---- LayerNorm backward + residual: lane has channels 16j + 4g + r of row m
+  // the LayerNorm's rows, behind the last product: lane part g of row `row`
+  // takes channels 16j + 4g + r
+  constexpr int NP = (4 * BM + 255) / 256;  // passes of 64 rows
+  float4 xr[NP][C / 16], dr[NP][C / 16];
+  float mu[NP], rs[NP];
+  const int part = tid & 3;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const long m = min(m0 + p * 64 + (tid >> 2), M - 1);
+#pragma unroll
+    for (int j = 0; j < C / 16; ++j) {
+      xr[p][j] = *reinterpret_cast<const float4*>(a.x + m * C + 16 * j + 4 * part);
+      dr[p][j] = *reinterpret_cast<const float4*>(a.dres + m * C + 16 * j + 4 * part);
+    }
+    mu[p] = a.mean[m];
+    rs[p] = a.rstd[m];
+  }
+#pragma unroll
+  for (int b = 0; b < KS; ++b)
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const h16x8 af = ld8(xs + (i * 16 + l16) * K::LDX + b * 32 + 8 * g);
+#pragma unroll
+      for (int jj = 0; jj < JJ; ++jj) acc2[i][jj] = mfma16x16x32(b2[b][jj], af, acc2[i][jj]);
+    }
+  __syncthreads();  // every wave is done with xs and hs, which T overlays
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int jj = 0; jj < JJ; ++jj)
+      *reinterpret_cast<f32x4*>(T + (i * 16 + l16) * K::LDT + 16 * (JJ * w + jj) + 4 * g) = acc2[i][jj];
+  __syncthreads();
+
+  // ---- LayerNorm backward + residual, four lanes a row
   const float gs = *a.gmul;
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const long m = m0 + i * 16 + l16;
-    const float mu = a.mean[m], rs = a.rstd[m];
+  for (int p = 0; p < NP; ++p) {
+    const int row = p * 64 + (tid >> 2);
+    const long m = m0 + row;
+    if (row >= BM || m >= M) continue;  // the row's four lanes leave together
     float xh[C / 16][4], gg[C / 16][4];
     float sg = 0.f, sgx = 0.f;
 #pragma unroll
     for (int j = 0; j < C / 16; ++j) {
-      const int c = 16 * j + 4 * g;
-      const float4 xv = xpre[i][j];
+      const int c = 16 * j + 4 * part;
+      const float4 dy = *reinterpret_cast<const float4*>(T + row * K::LDT + c);
       const float4 gm = *reinterpret_cast<const float4*>(a.ln_g + c);
-      const float xa[4] = {xv.x, xv.y, xv.z, xv.w}, ga[4] = {gm.x, gm.y, gm.z, gm.w};
+      const float xa[4] = {xr[p][j].x, xr[p][j].y, xr[p][j].z, xr[p][j].w};
+      const float ga[4] = {gm.x, gm.y, gm.z, gm.w}, da[4] = {dy.x, dy.y, dy.z, dy.w};
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        xh[j][r] = (xa[r] - mu) * rs;
-        gg[j][r] = acc2[i][j][r] * (ga[r] * gs);
+        xh[j][r] = (xa[r] - mu[p]) * rs[p];
+        gg[j][r] = da[r] * (ga[r] * gs);
         sg += gg[j][r];
         sgx += gg[j][r] * xh[j][r];
       }
     }
-    sg += __shfl_xor(sg, 16, 64);
-    sg += __shfl_xor(sg, 32, 64);
-    sgx += __shfl_xor(sgx, 16, 64);
-    sgx += __shfl_xor(sgx, 32, 64);
-    sg *= 1.f / C;
-    sgx *= 1.f / C;
+    sg = group_sum<4>(sg) * (1.f / C);
+    sgx = group_sum<4>(sgx) * (1.f / C);
 #pragma unroll
     for (int j = 0; j < C / 16; ++j) {
-      const int c = 16 * j + 4 * g;
-      const float4 d = *reinterpret_cast<const float4*>(a.dres + m * C + c);
       float4 o;
-      o.x = d.x + rs * (gg[j][0] - sg - xh[j][0] * sgx);
-      o.y = d.y + rs * (gg[j][1] - sg - xh[j][1] * sgx);
-      o.z = d.z + rs * (gg[j][2] - sg - xh[j][2] * sgx);
-      o.w = d.w + rs * (gg[j][3] - sg - xh[j][3] * sgx);
-      *reinterpret_cast<float4*>(a.out + m * C + c) = o;
+      o.x = dr[p][j].x + rs[p] * (gg[j][0] - sg - xh[j][0] * sgx);
+      o.y = dr[p][j].y + rs[p] * (gg[j][1] - sg - xh[j][1] * sgx);
+      o.z = dr[p][j].z + rs[p] * (gg[j][2] - sg - xh[j][2] * sgx);
+      o.w = dr[p][j].w + rs[p] * (gg[j][3] - sg - xh[j][3] * sgx);
+      *reinterpret_cast<float4*>(a.out + m * C + 16 * j + 4 * part) = o;
     }
   }
+}
+
+template <int C>
+void trimul_tail(hipStream_t st, const TailArgs& a) {
+  constexpr int RT = 3;
+  const long nwg = (a.M + 16 * RT - 1) / (16 * RT);
+  hipLaunchKernelGGL((trimul_tail_kernel<C, RT>), dim3(xcd_grid(nwg)), dim3(256), 0, st, a);
+}
+
+// The tail's weight fragments, 64 lanes x 8 binary16 each, lane 16 g + c, from
+// Wcat [C][NC]: GEMM1's ((j*4 + w)*2 + q)*KS + ks holds column 128j + 32w + 16q
+// + c at k = 32 ks + tail_k(g, e); GEMM2's (b*4 + w)*JJ + jj holds channel
+// 16 (JJ w + jj) + c at k = 32b + tail_k(g, e).
+std::vector<h16> tail_frags1(const std::vector<float>& cat, int C) {
+  const int NC = 5 * C, KS = C / 32;
+  std::vector<h16> f((size_t)4 * C * C);
+  size_t o = 0;
+  for (int jwq = 0; jwq < 4 * C / 16; ++jwq)
+    for (int ks = 0; ks < KS; ++ks)
+      for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e)
+          f[o++] = (h16)cat[(size_t)(32 * ks + tail_k(l >> 4, e)) * NC + 16 * jwq + (l & 15)];
+  return f;
+}
+std::vector<h16> tail_frags2(const std::vector<float>& cat, int C) {
+  const int NC = 5 * C;
+  std::vector<h16> f((size_t)NC * C);
+  size_t o = 0;
+  for (int b = 0; b < NC / 32; ++b)
+    for (int wj = 0; wj < C / 16; ++wj)
+      for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e)
+          f[o++] = (h16)cat[(size_t)(16 * wj + (l & 15)) * NC + 32 * b + tail_k(l >> 4, e)];
+  return f;
 }
 
 }  // namespace
@@ -603,17 +636,10 @@ TriMulW trimul_weights(WeightStore& ws, const std::string& P) {
       return b_frags_k128(NC, [&](int n, int k) { return c[(size_t)k * NC + n]; });
     });
   }
-  auto kperm_cols = [](std::vector<h16> m, int rows, int cols) {
-    std::vector<h16> o(m.size());
-    for (int r = 0; r < rows; ++r)
-      for (int p = 0; p < cols; ++p) o[(size_t)r * cols + p] = m[(size_t)r * cols + tail_kperm(p)];
-    return o;
-  };
-  w.wcat_k = ws.derived<h16>("trimul.wcat_k:" + P, [&] { return kperm_cols(to_h16(cat()), C, NC); });
-  w.wcat_tk = ws.derived<h16>("trimul.wcat_tk:" + P, [&] {
-    std::vector<float> c = cat();
-    return kperm_cols(transpose_h16(c.data(), C, NC), NC, C);
-  });
+  if (I == C && (C == 128 || C == 64)) {
+    w.tail_w1 = ws.derived<h16>("trimul.tail_w1:" + P, [&] { return tail_frags1(cat(), C); });
+    w.tail_w2 = ws.derived<h16>("trimul.tail_w2:" + P, [&] { return tail_frags2(cat(), C); });
+  }
   const HostTensor& ow = ws.host(P + "output_projection/weights");  // [I, C]
   w.wo = ws.derived<h16>("trimul.wo:" + P, [&] { return to_h16(ow.data); });
   w.wo_t = ws.derived<h16>("trimul.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), I, C); });
@@ -747,9 +773,9 @@ void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
   sc = module_scale(st, sc, dout, M * C);
-  // C = I = 128: the tail kernel keeps d(cat)'s [proj|gate] columns in
-  // registers; only its gating_linear columns ([M][C]) go through memory
-  const bool fused = (C == tail::C && I == tail::I && M % tail::BM == 0);
+  // I = C = 128 or 64: the tail kernel keeps d(cat)'s [proj|gate] columns on
+  // chip; only its gating_linear columns ([M][C]) go through memory
+  const bool fused = w.tail_w1 != nullptr;
   const int ldcat = fused ? C : NC, off = fused ? 0 : 4 * I;
   Sizer need;
   need.take<h16>((size_t)M * ldcat);  // dcat
@@ -811,14 +837,15 @@ void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   }
   if (fused) {
     TailArgs t;
-    t.xn = sv.xn; t.wcat_t = w.wcat_tk; t.wcat = w.wcat_k;
+    t.xn = sv.xn; t.w1 = w.tail_w1; t.w2 = w.tail_w2;
     t.dl = dL; t.dr = dR; t.dcg = dcat;
     t.bp = w.bp; t.bg = w.bg; t.mask = mask;
     t.x = pair_in; t.ln_g = w.ln_g; t.mean = sv.mean; t.rstd = sv.rstd; t.dres = dout;
     t.gmul = sc + 1;
     t.out = din; t.M = M;
     KTimed kt(BC2N_TN(C, "trimul.tail_bwd"), st);
-    hipLaunchKernelGGL(trimul_tail_kernel, dim3((unsigned)(M / tail::BM)), dim3(256), 0, st, t);
+    if (C == 128) trimul_tail<128>(st, t);
+    else trimul_tail<64>(st, t);
     return;
   }
   {
