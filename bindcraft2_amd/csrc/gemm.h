@@ -190,17 +190,8 @@ struct GemmSmem {
   static constexpr int BYTES = AB > T ? AB : T;
 };
 
-// An epilogue may ask for a minimum occupancy (kMinWaves waves per SIMD: the
-// register budget the compiler then keeps to), e.g. to fit a grid in one round.
-template <class E, class = void>
-struct epi_min_waves : std::integral_constant<int, 1> {};
-template <class E>
-struct epi_min_waves<E, std::void_t<decltype(E::kMinWaves)>>
-    : std::integral_constant<int, E::kMinWaves> {};
-
 template <int BM, int BN, int BK, bool AK, bool BKC, class Epi, class AL = ALoadDirect>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(epi_min_waves<Epi>::value)))
-void gemm_kernel(GemmArgs g, Epi epi, AL al = AL{}) {
+__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g, Epi epi, AL al = AL{}) {
   using SM = GemmSmem<BM, BN, BK>;
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
@@ -718,29 +709,6 @@ void gemm(hipStream_t st, const GemmArgs& g, const Epi& epi, const char* name = 
   gemm_launch<BM, BN>(st, g, epi, al);
 }
 
-// B operand of an N x 128 product (B(n, k), n < N, k < 128), N a multiple of
-// 128, rearranged for kernels that read B fragments straight from memory:
-// fragment ((j * 4 + w) * 2 + jj) * 4 + ks holds, at lane 16 g + c, the 8
-// values B(j*128 + 32w + 16jj + c, ks*32 + 8g + e), e = 0..7 -- the
-// v_mfma_f32_16x16x32_f16 B operand when A is K-contiguous -- so a wave
-// loads a fragment as one contiguous 1 KB.
-template <class B>
-std::vector<h16> b_frags_k128(int N, B b) {
-  std::vector<h16> f((size_t)N * 128);
-  for (int j = 0; j < N / 128; ++j)
-    for (int w = 0; w < 4; ++w)
-      for (int jj = 0; jj < 2; ++jj)
-        for (int ks = 0; ks < 4; ++ks)
-          for (int l = 0; l < 64; ++l)
-            for (int e = 0; e < 8; ++e)
-              f[((size_t)(((j * 4 + w) * 2 + jj) * 4 + ks) * 64 + l) * 8 + e] =
-                  (h16)b(j * 128 + 32 * w + 16 * jj + (l & 15), ks * 32 + 8 * (l >> 4) + e);
-  return f;
-}
-__device__ __forceinline__ h16x8 b_frag_k128(const h16* F, int j, int w, int jj, int ks, int lane) {
-  return ld8(F + ((long)(((j * 4 + w) * 2 + jj) * 4 + ks) * 64 + lane) * 8);
-}
-
 // ---------------------------------------------------------------- epilogues
 
 // C[b][m][n] = act(acc + bias[n]) (+= existing when ACC), OutT in {float, h16}.
@@ -808,22 +776,33 @@ struct EpiResidualRows : EpiRows {
   bool transpose;
   EpiResidualRows(const float* i, float* o, const float* b, const float* t, int n, int c, bool tr)
       : in(i), out(o), bias(b), tbl(t), nt(n), C(c), transpose(tr) {}
-  __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
-    const long src = transpose ? (long)(m % nt) * nt + m / nt : m;
-    float bb[8], x[8], r[8];
-    ld_f8(bias + n, bb);
+  struct Pre {
+    float bb[8], tt[8], r[8];
+    long o;
+  };
+  __device__ __forceinline__ void load(long m, int n, Pre& p) const {
+    const long src = transpose ? (long)((int)m % nt) * nt + (int)m / nt : m;
+    p.o = src * C + n;
+    ld_f8(bias + n, p.bb);
+    if (tbl) ld_f8(tbl + (long)((int)m % nt) * C + n, p.tt);
+    ld_f8(in + p.o, p.r);
+  }
+  __device__ __forceinline__ void row(long, int, const float (&v)[8], Pre& p) const {
+    float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = v[e] + bb[e];
+    for (int e = 0; e < 8; ++e) x[e] = v[e] + p.bb[e];
     if (tbl) {
-      float tt[8];
-      ld_f8(tbl + (long)(m % nt) * C + n, tt);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] *= tt[e];
+      for (int e = 0; e < 8; ++e) x[e] *= p.tt[e];
     }
-    ld_f8(in + src * C + n, r);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] += x[e];
-    st_f8(out + src * C + n, r);
+    for (int e = 0; e < 8; ++e) p.r[e] += x[e];
+    st_f8(out + p.o, p.r);
+  }
+  __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
+    Pre p;
+    load(m, n, p);
+    row((long)m, n, v, p);
   }
 };
 
@@ -831,8 +810,10 @@ struct EpiResidualRows : EpiRows {
 // d(og) = acc (og = o * sigmoid(g)):  dO = d(og) s,  dG = d(og) o s (1 - s),
 // s = sigmoid(g), and nDsum[r][h][q] = -(sum over head h's D columns of dO * o)
 // for token m = r * Ntok + q.  The D/8 row-mode calls of one head come from
-// consecutive lanes (8 columns each), which add their partials by DPP.
-struct EpiGateBwd : EpiRows {
+// consecutive lanes (8 columns each), which add their partials by DPP, or with
+// ACROSS from lanes 16 apart (lnproj.h): the same pairs in the same order.
+template <bool ACROSS>
+struct EpiGateBwdT : EpiRows {
   const h16* qkvg;  // gate pre-activation at column 3*HD + n of row m
   long ld;
   const h16* o;     // ungated attention output [M][HD]
@@ -841,30 +822,47 @@ struct EpiGateBwd : EpiRows {
   float* nDsum;      // [R][H][Ntok]
   int HD, H, D, Ntok;
   template <int W>
-  __device__ __forceinline__ float head_sum(float s) const { return group_sum<W>(s); }
-  __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
-    const h16x8 gv = ld8(qkvg + (long)m * ld + 3 * HD + n);
-    const h16x8 ov = ld8(o + (long)m * HD + n);
+  __device__ __forceinline__ float head_sum(float s) const {
+    if constexpr (!ACROSS) return group_sum<W>(s);
+    s += __shfl_xor(s, 16, 64);
+    if constexpr (W == 4) s += __shfl_xor(s, 32, 64);
+    return s;
+  }
+  struct Pre {
+    h16x8 gv, ov;
+  };
+  __device__ __forceinline__ void load(long m, int n, Pre& p) const {
+    p.gv = ld8(qkvg + m * ld + 3 * HD + n);
+    p.ov = ld8(o + m * HD + n);
+  }
+  __device__ __forceinline__ void row(long m, int n, const float (&v)[8], const Pre& p) const {
     h16x8 dov, dgv;
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float sg = sigmoidf_((float)gv[e]);
-      const float oo = (float)ov[e];
+      const float sg = sigmoidf_((float)p.gv[e]);
+      const float oo = (float)p.ov[e];
       const float d = v[e] * sg;
       dov[e] = f2h_sat(d);
       dgv[e] = f2h_sat(v[e] * oo * sg * (1.f - sg));
       s += d * oo;
     }
-    st8(dO + (long)m * HD + n, dov);
-    st8(dqkvg + (long)m * ld + 3 * HD + n, dgv);
+    st8(dO + m * HD + n, dov);
+    st8(dqkvg + m * ld + 3 * HD + n, dgv);
     s = D == 32 ? head_sum<4>(s) : head_sum<2>(s);
     if (n % D == 0) {
-      const int r = m / Ntok, q = m % Ntok;
+      const int r = (int)m / Ntok, q = (int)m % Ntok;
       nDsum[((long)r * H + n / D) * Ntok + q] = -s;
     }
   }
+  __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
+    Pre p;
+    load(m, n, p);
+    row((long)m, n, v, p);
+  }
 };
+
+using EpiGateBwd = EpiGateBwdT<false>;
 
 // dH = acc * (H > 0): backward through a ReLU of the kept tensor H (h16
 // or binary16).

@@ -33,8 +33,8 @@ struct TriAttnW {
   const float *ln_g = nullptr, *ln_b = nullptr, *w2d = nullptr;  // w2d [C][H]
   const float* bqkvg = nullptr;  // [4HD]: zeros for q,k,v; gating_b for g
   const h16* wqkvg_t = nullptr; // [4HD][C]
-  const h16* wqkvg_frag = nullptr;  // C = 128: wqkvg_t in b_frags_k128 order
-  const h16* wo_frag = nullptr;     // C = HD = 128: wo_t in b_frags_k128 order
+  // C = 128 or 64, H = 4: wqkvg_t, wo_t and wo in proj_frags order
+  const h16 *wqkvg_frag = nullptr, *wo_frag = nullptr, *wo_bfrag = nullptr;
   const h16* wqkvg = nullptr;   // [C][4HD]
   const h16* wo_t = nullptr;    // [C][HD]
   const h16* wo = nullptr;      // [HD][C]
@@ -66,9 +66,9 @@ struct TriMulW {
   const float *bp = nullptr, *bg = nullptr, *bgl = nullptr, *bo = nullptr;
   const h16* wcat = nullptr;    // [C][4I+C]  (GEMM column order)
   const h16* wcat_t = nullptr;  // [4I+C][C]
-  const h16* wcat_frag = nullptr;  // C = 128: wcat_t in b_frags_k128 order
-  const h16* wo_frag = nullptr;    // C = I = 128: wo_t in b_frags_k128 order
-  // I = C = 128 or 64: both products of the backward tail in its fragment order
+  // I = C = 128 or 64: wcat_t, wo_t and wo in proj_frags order, and both
+  // products of the backward tail in its own
+  const h16 *wcat_frag = nullptr, *wo_frag = nullptr, *wo_bfrag = nullptr;
   const h16 *tail_w1 = nullptr, *tail_w2 = nullptr;
   const h16* wo = nullptr;      // [I][C]
   const h16* wo_t = nullptr;    // [C][I]

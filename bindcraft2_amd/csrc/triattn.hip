@@ -72,10 +72,11 @@ TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
     std::vector<float> c = cat();
     return transpose_h16(c.data(), C, 4 * HD);
   });
-  if (C == 128 && w.H == 4 && (4 * HD) % 128 == 0) {
+  const bool rows = (C == 128 || C == 64) && w.H == 4;  // the row-tile kernels' widths
+  if (rows) {
     w.wqkvg_frag = ws.derived<h16>("triattn.wqkvg_frag:" + P, [&] {
       const std::vector<float> c = cat();  // [C][4HD]
-      return b_frags_k128(4 * HD, [&](int n, int k) { return c[(size_t)k * 4 * HD + n]; });
+      return proj_frags(4 * HD, C, 0, [&](int n, int k) { return c[(size_t)k * 4 * HD + n]; });
     });
   }
   w.bqkvg = ws.derived<float>("triattn.bqkvg:" + P, [&] {
@@ -88,9 +89,12 @@ TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
   w.wo = ws.derived<h16>("triattn.wo:" + P, [&] { return to_h16(ow.data); });
   w.wo_t = ws.derived<h16>("triattn.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), HD, C); });
   w.bo = ws.f32(P + "attention/output_b");
-  if (C == 128 && HD == 128) {
+  if (rows) {
     w.wo_frag = ws.derived<h16>("triattn.wo_frag:" + P, [&] {
-      return b_frags_k128(C, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
+      return proj_frags(C, HD, 0, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
+    });
+    w.wo_bfrag = ws.derived<h16>("triattn.wo_bfrag:" + P, [&] {
+      return proj_frags(HD, C, 0, [&](int n, int k) { return ow.data[(size_t)n * C + k]; });
     });
   }
   return w;
@@ -125,8 +129,9 @@ static void triattn_fwd_with(hipStream_t st, const TriAttnW& w, bool per_column,
     // xn stays on chip: the backward's LayerNorm term reads pair_in, mean and rstd
     la.xn = nullptr; la.mean = sv.mean; la.rstd = sv.rstd; la.bias = sv.bias; la.W = w.wqkvg_frag;
     KTimed kt(BC2N_TN(C, "triattn.ln_qkvg"), st);
-    if (H != 4) throw std::runtime_error("triattn: the fused LayerNorm-projection takes 4 bias heads");
-    lnproj::launch<4, false>(st, la, EpiScaledCols(sv.qkvg, 4L * HD, w.bqkvg, qscale, HD));
+    const EpiScaledCols cols(sv.qkvg, 4L * HD, w.bqkvg, qscale, HD);
+    if (C == 128) lnproj::launch<lnproj::In::LN, 128, 4, false>(st, la, cols);
+    else lnproj::launch<lnproj::In::LN, 64, 4, false>(st, la, cols);
   } else {
     {
       KTimed kt(BC2N_TN(C, "triattn.ln_fwd"), st);
@@ -157,7 +162,8 @@ static void triattn_fwd_with(hipStream_t st, const TriAttnW& w, bool per_column,
     lnproj::Args la{};
     la.M = M; la.nout = C; la.xn = og; la.W = w.wo_frag;
     KTimed kt(BC2N_TN(C, "triattn.gemm_out"), st);
-    lnproj::launch_rows(st, la, res);
+    if (C == 128) lnproj::launch<lnproj::In::ROWS, 128, 0, false>(st, la, res);
+    else lnproj::launch<lnproj::In::ROWS, 64, 0, false>(st, la, res);
     return;
   }
   GemmArgs g2;
@@ -260,17 +266,27 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
 
   // d(og) = (tbl * dout) . Wo^T, the dropout scale applied as A is loaded;
   // the epilogue continues through the gate (dO, dG, Dsum)
-  GemmArgs g1;
-  g1.M = (int)M; g1.N = HD; g1.K = C;
-  g1.a_sm = C; g1.a_sk = 1;
-  g1.B = w.wo; g1.b_sn = C; g1.b_sk = 1;
-  EpiGateBwd eg;
-  eg.qkvg = sv.qkvg; eg.ld = 4L * HD; eg.o = sv.o; eg.dO = b.dO; eg.dqkvg = b.dqkvg;
-  eg.nDsum = b.nDsum; eg.HD = HD; eg.H = H; eg.D = w.D; eg.Ntok = N;
-  // 64-row tiles: with N = K = 128 a 128-row grid leaves most workgroup
-  // slots empty (392 workgroups at 224 tokens); the 128 x 128 B operand is
-  // cheap to re-read
-  gemm<64, 128>(st, g1, eg, BC2N_TN(C, "triattn.gemm_dout"), ALoadScaledRows{dout, tbl, N, C, per_column, sc});
+  auto gate = [&](auto eg) {
+    eg.qkvg = sv.qkvg; eg.ld = 4L * HD; eg.o = sv.o; eg.dO = b.dO; eg.dqkvg = b.dqkvg;
+    eg.nDsum = b.nDsum; eg.HD = HD; eg.H = H; eg.D = w.D; eg.Ntok = N;
+    return eg;
+  };
+  if (w.wo_bfrag) {
+    lnproj::Args la{};
+    la.M = M; la.nt = per_column ? N : 0; la.bn = N; la.nout = HD;
+    la.x = dout; la.tbl = tbl; la.sc = sc; la.W = w.wo_bfrag;
+    KTimed kt(BC2N_TN(C, "triattn.gemm_dout"), st);
+    const auto eg = gate(EpiGateBwdT<true>{});
+    if (C == 128) lnproj::launch<lnproj::In::SCALED, 128, 0, false>(st, la, eg);
+    else lnproj::launch<lnproj::In::SCALED, 64, 0, false>(st, la, eg);
+  } else {
+    GemmArgs g1;
+    g1.M = (int)M; g1.N = HD; g1.K = C;
+    g1.a_sm = C; g1.a_sk = 1;
+    g1.B = w.wo; g1.b_sn = C; g1.b_sk = 1;
+    gemm<64, 128>(st, g1, gate(EpiGateBwd{}), BC2N_TN(C, "triattn.gemm_dout"),
+                  ALoadScaledRows{dout, tbl, N, C, per_column, sc});
+  }
   b.gate_done = true;
 
   AttnArgs& a = b.f;

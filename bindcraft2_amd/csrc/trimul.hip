@@ -39,7 +39,6 @@ __host__ __device__ inline int col_gate(int ch) { return (ch / 16) * 32 + 16 + c
 // gating_linear columns run in row mode: g_out[m][c] = sigmoid(acc + b).
 struct EpiTrimulProj {
   static constexpr bool kHasCol = true;
-  static constexpr bool kColPairs = true;  // col() of column c also does its gate c + 16
   h16 *left, *right;   // [I][M]
   h16* gout;           // [M][C]
   const float *bp, *bg, *bgl, *mask;
@@ -62,6 +61,16 @@ struct EpiTrimulProj {
     }
     if (ch < I) st_h8f(left + (long)ch * M + m, av);
     else st_h8f(right + (long)(ch - I) * M + m, av);
+  }
+  // 8 rows m.. of projection column n and of its gate (lnproj.h)
+  __device__ __forceinline__ void cols(long m, int n, float (&pv)[8], const float (&gv)[8]) const {
+    const int ch = (n >> 5) * 16 + (n & 15);
+    const float bpv = bp[ch], bgv = bg[ch];
+    float mk[8];
+    ld_f8(mask + m, mk);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) pv[e] = mk[e] * (pv[e] + bpv) * sigmoidf_(gv[e] + bgv);
+    st_h8f((ch < I ? left + (long)ch * M : right + (long)(ch - I) * M) + m, pv);
   }
   __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
     const int c = n - 4 * I;
@@ -86,26 +95,37 @@ struct EpiTrimulOut : EpiRows {
   EpiTrimulOut(const float* i, float* o, const float* b, const h16* g, h16* os, const float* t,
                int n, int c)
       : in(i), out(o), bo(b), gout(g), osave(os), tbl(t), nt(n), C(c) {}
-  __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
-    const long o = (long)m * C + n;
-    float bb[8], ov[8], gv[8], r[8];
-    ld_f8(bo + n, bb);
+  struct Pre {
+    float bb[8], tt[8], r[8];
+    h16x8 gv;
+  };
+  __device__ __forceinline__ void load(long m, int n, Pre& p) const {
+    const long o = m * C + n;
+    ld_f8(bo + n, p.bb);
+    p.gv = ld8(gout + o);
+    if (tbl) ld_f8(tbl + (long)((int)m % nt) * C + n, p.tt);
+    ld_f8(in + o, p.r);
+  }
+  __device__ __forceinline__ void row(long m, int n, const float (&v)[8], Pre& p) const {
+    const long o = m * C + n;
+    float ov[8], gv[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ov[e] = v[e] + bb[e];
+    for (int e = 0; e < 8; ++e) ov[e] = v[e] + p.bb[e];
     st_h8f(osave + o, ov);
-    ld_h8f(gout + o, gv);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) gv[e] *= ov[e];
+    for (int e = 0; e < 8; ++e) gv[e] = (float)p.gv[e] * ov[e];
     if (tbl) {
-      float tt[8];
-      ld_f8(tbl + (long)(m % nt) * C + n, tt);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) gv[e] *= tt[e];
+      for (int e = 0; e < 8; ++e) gv[e] *= p.tt[e];
     }
-    ld_f8(in + o, r);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] += gv[e];
-    st_f8(out + o, r);
+    for (int e = 0; e < 8; ++e) p.r[e] += gv[e];
+    st_f8(out + o, p.r);
+  }
+  __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
+    Pre p;
+    load(m, n, p);
+    row((long)m, n, v, p);
   }
 };
 
@@ -206,73 +226,77 @@ struct ALoadTrimulOut {
   }
 };
 
-// The centre LayerNorm's backward fused into the d(tn) product as its
-// row-block epilogue (I = 128): each staged half tile of d(tn) rows is the dy
-// of ln_bwd_cm, normalised with the same arithmetic in the same order (eight
-// lanes a row, 16 consecutive channels each, the x values read from the
-// channel-major T), and written channel-major in binary16 through the tile,
-// so d(tn) never reaches memory.
+// The centre LayerNorm's backward fused into the d(tn) product (I = C): the
+// staged tile of d(tn) rows is the dy of ln_bwd_cm, normalised with the same
+// sums in the same order (eight parts a row, C / 8 consecutive channels each),
+// and written channel-major in binary16, so d(tn) never reaches memory.  A
+// lane is a row and a wave one or two parts, so that the channel-major T is
+// read (before the product) and dT written 64 or 32 rows of a channel at a
+// time; the parts' sums meet in LDS.
+template <int C_>
 struct EpiCmLnBwd : EpiRows {
-  static constexpr bool kRowBlock = true;
-  // four waves a SIMD: the 64-row grid (784 workgroups at 224 tokens) in one
-  // round of 1024 slots (three would leave 16 workgroups for a second round)
-  static constexpr int kMinWaves = 4;
-  static constexpr int C = 128, P = 8, CPL = C / P;
+  static constexpr int C = C_, P = 8, CPL = C / P;
   const float *x, *gamma, *mean, *rstd;  // x: channel-major [C][M]
   h16* dx;                               // channel-major [C][M]
   long M;
-  static constexpr int WMP = 256 / P;  // rows a pass: one (of eight lanes) a thread
-  __device__ __forceinline__ void row(int, int, int, const float (&)[8]) const {}
-  template <int WM>
-  __device__ __forceinline__ void block(int, long mb, const float* T, int ldt, int tid) const {
-    static_assert(WM == WMP, "one 32-row pass a call");
-    float* Tw = const_cast<float*>(T);  // the kernel's own staging tile
-    {
-      const int r = tid / P, part = tid % P;
-      const long m = mb + r;
-      const bool live = m < M;
-      const float mu = live ? mean[m] : 0.f, rs = live ? rstd[m] : 0.f;
-      float xv[CPL];
+  struct Tile {
+    float x[2 * CPL], mu, rs;
+  };
+  template <int BM>
+  static constexpr int parts() { return P * BM / 256; }  // a thread's parts
+  template <int BM>
+  __device__ __forceinline__ void load(long m0, Tile& t, int tid) const {
+    const long m = min(m0 + tid % BM, M - 1);  // rows past M: never stored
 #pragma unroll
-      for (int e = 0; e < CPL; ++e) xv[e] = live ? x[(long)(part * CPL + e) * M + m] : 0.f;
-      float xh[CPL], g[CPL];
+    for (int k = 0; k < parts<BM>(); ++k)
+#pragma unroll
+      for (int e = 0; e < CPL; ++e)
+        t.x[k * CPL + e] = x[(long)((tid / BM + 256 / BM * k) * CPL + e) * M + m];
+    t.mu = mean[m];
+    t.rs = rstd[m];
+  }
+  template <int BM>
+  __device__ __forceinline__ void tile(long m0, const float* T, int ldt, int tid, Tile& t) const {
+    __shared__ float red[2][P][BM];
+    const int r = tid % BM;
+    float g[parts<BM>() * CPL];
+#pragma unroll
+    for (int k = 0; k < parts<BM>(); ++k) {
+      const int part = tid / BM + 256 / BM * k;
       float sg = 0.f, sgx = 0.f;
 #pragma unroll
       for (int e0 = 0; e0 < CPL; e0 += 4) {
-        float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (live) d = *reinterpret_cast<const float4*>(T + r * ldt + part * CPL + e0);
+        const float4 d = *reinterpret_cast<const float4*>(T + r * ldt + part * CPL + e0);
         const float dv[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int e = e0 + k, c = part * CPL + e;
-          xh[e] = (xv[e] - mu) * rs;
-          g[e] = dv[k] * gamma[c];
-          sg += g[e];
-          sgx += g[e] * xh[e];
+        for (int q = 0; q < 4; ++q) {
+          const int i = k * CPL + e0 + q;
+          t.x[i] = (t.x[i] - t.mu) * t.rs;
+          g[i] = dv[q] * gamma[part * CPL + e0 + q];
+          sg += g[i];
+          sgx += g[i] * t.x[i];
         }
       }
-      sg = group_sum<P>(sg) / C;
-      sgx = group_sum<P>(sgx) / C;
-      // each thread rewrites exactly the 16 values it read
-#pragma unroll
-      for (int e = 0; e < CPL; ++e) {
-        const int c = part * CPL + e;
-        Tw[r * ldt + c] = rs * (g[e] - sg - xh[e] * sgx);
-      }
+      red[0][part][r] = sg;
+      red[1][part][r] = sgx;
     }
     __syncthreads();
-    for (int i = tid; i < C * (WM / 4); i += 256) {
-      const int c = i / (WM / 4), q = (i % (WM / 4)) * 4;
-      const long mm = mb + q;
-      if (mm < M) {
-        h16x4 o;
-        o[0] = f2h_sat(T[(q + 0) * ldt + c]);
-        o[1] = f2h_sat(T[(q + 1) * ldt + c]);
-        o[2] = f2h_sat(T[(q + 2) * ldt + c]);
-        o[3] = f2h_sat(T[(q + 3) * ldt + c]);
-        *reinterpret_cast<h16x4*>(dx + (long)c * M + mm) = o;
+    auto total = [&](int q) {  // group_sum<8>'s pairs
+      float v[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) v[p] = red[q][p][r];
+      return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    };
+    const float sg = total(0) / C, sgx = total(1) / C;
+    if (m0 + r >= M) return;
+#pragma unroll
+    for (int k = 0; k < parts<BM>(); ++k)
+#pragma unroll
+      for (int e = 0; e < CPL; ++e) {
+        const int i = k * CPL + e;
+        dx[(long)((tid / BM + 256 / BM * k) * CPL + e) * M + m0 + r] =
+            f2h_sat(t.rs * (g[i] - sg - t.x[i] * sgx));
       }
-    }
   }
 };
 
@@ -630,22 +654,24 @@ TriMulW trimul_weights(WeightStore& ws, const std::string& P) {
     std::vector<float> c = cat();
     return transpose_h16(c.data(), C, NC);
   });
-  if (C == 128 && NC % 128 == 0) {
+  const bool rows = I == C && (C == 128 || C == 64);  // the row-tile kernels' widths
+  if (rows) {
     w.wcat_frag = ws.derived<h16>("trimul.wcat_frag:" + P, [&] {
       const std::vector<float> c = cat();  // [C][NC]
-      return b_frags_k128(NC, [&](int n, int k) { return c[(size_t)k * NC + n]; });
+      return proj_frags(NC, C, 4 * I, [&](int n, int k) { return c[(size_t)k * NC + n]; });
     });
-  }
-  if (I == C && (C == 128 || C == 64)) {
     w.tail_w1 = ws.derived<h16>("trimul.tail_w1:" + P, [&] { return tail_frags1(cat(), C); });
     w.tail_w2 = ws.derived<h16>("trimul.tail_w2:" + P, [&] { return tail_frags2(cat(), C); });
   }
   const HostTensor& ow = ws.host(P + "output_projection/weights");  // [I, C]
   w.wo = ws.derived<h16>("trimul.wo:" + P, [&] { return to_h16(ow.data); });
   w.wo_t = ws.derived<h16>("trimul.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), I, C); });
-  if (C == 128 && I == 128) {
+  if (rows) {
     w.wo_frag = ws.derived<h16>("trimul.wo_frag:" + P, [&] {
-      return b_frags_k128(C, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
+      return proj_frags(C, I, 0, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
+    });
+    w.wo_bfrag = ws.derived<h16>("trimul.wo_bfrag:" + P, [&] {
+      return proj_frags(I, C, 0, [&](int n, int k) { return ow.data[(size_t)n * C + k]; });
     });
   }
   return w;
@@ -717,7 +743,8 @@ void trimul_fwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
     la.x = pair_in; la.g = w.ln_g; la.b = w.ln_b;
     la.xn = xn; la.mean = sv.mean; la.rstd = sv.rstd; la.W = w.wcat_frag;
     KTimed kt(BC2N_TN(C, "trimul.ln_proj"), st);
-    lnproj::launch<0, true>(st, la, proj);
+    if (C == 128) lnproj::launch<lnproj::In::LN, 128, 0, true>(st, la, proj);
+    else lnproj::launch<lnproj::In::LN, 64, 0, true>(st, la, proj);
   } else {
     {
       KTimed kt(BC2N_TN(C, "trimul.ln_fwd"), st);
@@ -732,26 +759,20 @@ void trimul_fwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   }
   contraction_fwd(st, outgoing, N, I, sv.left, sv.right, sv.T);
   const EpiTrimulOut out(pair_in, pair_out, w.bo, sv.gout, sv.osave, tbl, N, C);
-  if (w.wo_frag && I == lnproj::C) {
+  if (w.wo_frag) {
     // the centre norm and the output projection in one kernel: the normalised
     // rows stay on chip (the same statistics and binary16 rows as ln_fwd_cm)
     lnproj::Args la{};
     la.M = M; la.nout = C; la.x = sv.T; la.g = w.cn_g; la.b = w.cn_b;
     la.mean = sv.cmean; la.rstd = sv.crstd; la.W = w.wo_frag;
     KTimed kt(BC2N_TN(C, "trimul.ln_out"), st);
-    lnproj::launch_cm<true>(st, la, out);
+    if (C == 128) lnproj::launch<lnproj::In::CM, 128, 0, true>(st, la, out);
+    else lnproj::launch<lnproj::In::CM, 64, 0, true>(st, la, out);
     return;
   }
   {
     KTimed kt(BC2N_TN(C, "trimul.ln_center"), st);
     ln_fwd_cm(st, sv.T, M, I, w.cn_g, w.cn_b, tn, sv.cmean, sv.crstd, true);
-  }
-  if (w.wo_frag) {
-    lnproj::Args la{};
-    la.M = M; la.nout = C; la.xn = tn; la.W = w.wo_frag;
-    KTimed kt(BC2N_TN(C, "trimul.gemm_out"), st);
-    lnproj::launch_rows(st, la, out);
-    return;
   }
   GemmArgs g2;
   g2.M = (int)M; g2.N = C; g2.K = I;
@@ -779,37 +800,40 @@ void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   const int ldcat = fused ? C : NC, off = fused ? 0 : 4 * I;
   Sizer need;
   need.take<h16>((size_t)M * ldcat);  // dcat
-  need.take<float>((size_t)M * I);  // dTn
+  if (!fused) need.take<float>((size_t)M * I);  // dTn
   need.take<h16>((size_t)M * I);   // dT
   need.take<h16>((size_t)M * I);   // dL
   need.take<h16>((size_t)M * I);   // dR
   if (!fused) need.take<float>((size_t)M * C);  // dxn
   ar.reset(st, need.off);
   h16* dcat = ar.take_n<h16>((size_t)M * ldcat);
-  float* dtn = ar.take_n<float>((size_t)M * I);
+  float* dtn = fused ? nullptr : ar.take_n<float>((size_t)M * I);
   h16* dT = ar.take_n<h16>((size_t)M * I);
   h16* dL = ar.take_n<h16>((size_t)M * I);
   h16* dR = ar.take_n<h16>((size_t)M * I);
   float* dxn = fused ? nullptr : ar.take_n<float>((size_t)M * C);
 
-  // d(tn) = (tbl*dout*g_out) . Wo^T, the operand built as the GEMM loads it;
-  // the loader also writes the gating_linear columns of dcat
-  GemmArgs g1;
-  g1.M = (int)M; g1.N = I; g1.K = C;
-  g1.a_sm = C; g1.a_sk = 1;
-  g1.B = w.wo; g1.b_sn = C; g1.b_sk = 1;
-  // 64-row tiles: with N = K = 128 a 128-row grid leaves most workgroup
-  // slots empty (392 workgroups at 224 tokens); the 128 x 128 B operand is
-  // cheap to re-read
-  const ALoadTrimulOut aload{dout, tbl, sv.gout, sv.osave, dcat, C, ldcat, off, N, sc};
-  if (I == EpiCmLnBwd::C && M % 4 == 0) {
+  // d(tn) = (tbl*dout*g_out) . Wo^T, the operand built as the product loads
+  // it, which also writes the gating_linear columns of dcat
+  if (fused) {
     // the centre norm's backward in the epilogue: dT straight from d(tn)
-    EpiCmLnBwd ep;
-    ep.x = sv.T; ep.gamma = w.cn_g; ep.mean = sv.cmean; ep.rstd = sv.crstd; ep.dx = dT; ep.M = M;
-    gemm<64, 128>(st, g1, ep, BC2N_TN(C, "trimul.gemm_dout_ln"), aload);
+    lnproj::Args la{};
+    la.M = M; la.bn = N; la.nout = I; la.x = dout; la.tbl = tbl; la.sc = sc;
+    la.gout = sv.gout; la.osave = sv.osave; la.dcat = dcat; la.W = w.wo_bfrag;
+    KTimed kt(BC2N_TN(C, "trimul.gemm_dout_ln"), st);
+    auto go = [&](auto ep) {
+      ep.x = sv.T; ep.gamma = w.cn_g; ep.mean = sv.cmean; ep.rstd = sv.crstd; ep.dx = dT; ep.M = M;
+      lnproj::launch<lnproj::In::GATED, decltype(ep)::C, 0, false>(st, la, ep);
+    };
+    if (C == 128) go(EpiCmLnBwd<128>{});
+    else go(EpiCmLnBwd<64>{});
   } else {
+    GemmArgs g1;
+    g1.M = (int)M; g1.N = I; g1.K = C;
+    g1.a_sm = C; g1.a_sk = 1;
+    g1.B = w.wo; g1.b_sn = C; g1.b_sk = 1;
     gemm<64, 128>(st, g1, EpiStore<float>{dtn, I, 0, nullptr, I}, BC2N_TN(C, "trimul.gemm_dout"),
-                  aload);
+                  ALoadTrimulOut{dout, tbl, sv.gout, sv.osave, dcat, C, ldcat, off, N, sc});
     KTimed kt(BC2N_TN(C, "trimul.ln_center_bwd"), st);
     ln_bwd_cm(st, dtn, sv.T, M, I, w.cn_g, sv.cmean, sv.crstd, dT);
   }
