@@ -46,6 +46,17 @@ __device__ __forceinline__ void st_f8(float* p, const float (&v)[8]) {
   reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
   reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
 }
+// p[0..3] and p[d..d+3]
+__device__ __forceinline__ void ld_f44(const float* p, int d, float (&v)[8]) {
+  const float4 a = *reinterpret_cast<const float4*>(p);
+  const float4 b = *reinterpret_cast<const float4*>(p + d);
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void st_f44(float* p, int d, const float (&v)[8]) {
+  *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+  *reinterpret_cast<float4*>(p + d) = make_float4(v[4], v[5], v[6], v[7]);
+}
 __device__ __forceinline__ void ld_h8f(const h16* p, float (&v)[8]) {
   const h16x8 a = ld8(p);
 #pragma unroll
@@ -776,18 +787,21 @@ struct EpiResidualRows : EpiRows {
   bool transpose;
   EpiResidualRows(const float* i, float* o, const float* b, const float* t, int n, int c, bool tr)
       : in(i), out(o), bias(b), tbl(t), nt(n), C(c), transpose(tr) {}
+  // lnproj.h: columns n..n+3 and n+d..n+d+3 a call (f32 rows are best read and
+  // written 16 bytes a lane, 64 a row)
+  static constexpr bool kQuads = true;
   struct Pre {
     float bb[8], tt[8], r[8];
     long o;
   };
-  __device__ __forceinline__ void load(long m, int n, Pre& p) const {
+  __device__ __forceinline__ void load(long m, int n, Pre& p, int d) const {
     const long src = transpose ? (long)((int)m % nt) * nt + (int)m / nt : m;
     p.o = src * C + n;
-    ld_f8(bias + n, p.bb);
-    if (tbl) ld_f8(tbl + (long)((int)m % nt) * C + n, p.tt);
-    ld_f8(in + p.o, p.r);
+    ld_f44(bias + n, d, p.bb);
+    if (tbl) ld_f44(tbl + (long)((int)m % nt) * C + n, d, p.tt);
+    ld_f44(in + p.o, d, p.r);
   }
-  __device__ __forceinline__ void row(long, int, const float (&v)[8], Pre& p) const {
+  __device__ __forceinline__ void row(long, int, const float (&v)[8], Pre& p, int d) const {
     float x[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = v[e] + p.bb[e];
@@ -797,12 +811,12 @@ struct EpiResidualRows : EpiRows {
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) p.r[e] += x[e];
-    st_f8(out + p.o, p.r);
+    st_f44(out + p.o, d, p.r);
   }
   __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
     Pre p;
-    load(m, n, p);
-    row((long)m, n, v, p);
+    load(m, n, p, 4);
+    row((long)m, n, v, p, 4);
   }
 };
 
@@ -831,11 +845,11 @@ struct EpiGateBwdT : EpiRows {
   struct Pre {
     h16x8 gv, ov;
   };
-  __device__ __forceinline__ void load(long m, int n, Pre& p) const {
+  __device__ __forceinline__ void load(long m, int n, Pre& p, int) const {
     p.gv = ld8(qkvg + m * ld + 3 * HD + n);
     p.ov = ld8(o + m * HD + n);
   }
-  __device__ __forceinline__ void row(long m, int n, const float (&v)[8], const Pre& p) const {
+  __device__ __forceinline__ void row(long m, int n, const float (&v)[8], const Pre& p, int) const {
     h16x8 dov, dgv;
     float s = 0.f;
 #pragma unroll
@@ -857,8 +871,8 @@ struct EpiGateBwdT : EpiRows {
   }
   __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
     Pre p;
-    load(m, n, p);
-    row((long)m, n, v, p);
+    load(m, n, p, 4);
+    row((long)m, n, v, p, 4);
   }
 };
 

@@ -88,12 +88,18 @@ __host__ __device__ constexpr int row_of(int p) {
 }
 
 // An epilogue with operands of its own (nout == C) declares struct Pre,
-// load(m, n, pre) and row(m, n, v, pre): the loads of all of a lane's rows are
-// then in flight together.
+// load(m, n, pre, d) and row(m, n, v, pre, d), for columns n..n+3 and
+// n+d..n+d+3 of a row: the loads of all of a lane's rows are then in flight
+// together.  With kQuads its weights are in column-mode order and d is 16.
 template <class E, class = void>
 struct has_pre : std::false_type {};
 template <class E>
 struct has_pre<E, std::void_t<typename E::Pre>> : std::true_type {};
+
+template <class E, class = void>
+struct quads : std::false_type {};
+template <class E>
+struct quads<E, std::void_t<decltype(E::kQuads)>> : std::bool_constant<E::kQuads> {};
 
 template <class E, class = void>
 struct has_tile : std::false_type {};
@@ -377,16 +383,18 @@ kernel(Args a, Epi epi) {
       __syncthreads();
       epi.template tile<BM>(m0, T, LDT, tid, tl);
     } else if constexpr (has_pre<Epi>::value) {
+      constexpr bool Q = quads<Epi>::value;
+      const int n = n0 + (Q ? 4 : 8) * g;
       typename Epi::Pre pre[TI];
 #pragma unroll
-      for (int i = 0; i < TI; ++i) epi.load(min(row_m(i), M - 1), n0 + 8 * g, pre[i]);
+      for (int i = 0; i < TI; ++i) epi.load(min(row_m(i), M - 1), n, pre[i], Q ? 16 : 4);
 #pragma unroll
       for (int i = 0; i < TI; ++i) {
         const long m = row_m(i);
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = acc[i][e / 4][e % 4];
-        if (m < M) epi.row(m, n0 + 8 * g, v, pre[i]);
+        if (m < M) epi.row(m, n, v, pre[i], Q ? 16 : 4);
       }
     } else {
 #pragma unroll
@@ -409,7 +417,9 @@ kernel(Args a, Epi epi) {
 // 196 / 117 (trimul's); CM at M = 65536 26 / 27, 173056 84 / 80, 262144 132 /
 // 122; GATED at M = 65536 21 / 21, 102400 40 / 37, 262144 106 / 98.  SCALED
 // (14 / 17 at 50176, 79 / 77 at 262144) keeps 32; ROWS takes 48 beyond 32768
-// (8.0 against 9.3 at 36864, 72 against 74 at 262144).
+// (8.0 against 9.3 at 36864, 72 against 74 at 262144).  Triangle attention's LN
+// takes 48 where 64-row workgroups come to one round and a little, or to much
+// less than one (18.1 against 20.6 at 36864, 26.5 / 27.3 at 50176; 33 / 30 at 65536).
 template <In IN, int C, int H, bool FAST, class Epi>
 void launch(hipStream_t st, const Args& a, const Epi& epi) {
   static_assert(H == 0 || H == 4, "bias heads 0 or 4");
@@ -442,6 +452,12 @@ void launch(hipStream_t st, const Args& a, const Epi& epi) {
     }
   } else {
     constexpr long tall = IN == In::LN ? 64 : IN == In::CM ? 512 : 288;
+    if constexpr (C == 128 && IN == In::LN && !Epi::kHasCol) {
+      if (per_cu > 112 && per_cu < 224) {
+        width(integral_constant<int, 3>());
+        return;
+      }
+    }
     if (per_cu >= tall) width(integral_constant<int, 4>());
     else width(integral_constant<int, 2>());
   }

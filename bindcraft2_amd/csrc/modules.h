@@ -33,8 +33,9 @@ struct TriAttnW {
   const float *ln_g = nullptr, *ln_b = nullptr, *w2d = nullptr;  // w2d [C][H]
   const float* bqkvg = nullptr;  // [4HD]: zeros for q,k,v; gating_b for g
   const h16* wqkvg_t = nullptr; // [4HD][C]
-  // C = 128 or 64, H = 4: wqkvg_t, wo_t and wo in proj_frags order
-  const h16 *wqkvg_frag = nullptr, *wo_frag = nullptr, *wo_bfrag = nullptr;
+  // C = 128 or 64, H = 4: wqkvg_t, wo_t and wo in proj_frags order, wqkvg in
+  // the backward's dX kernel's
+  const h16 *wqkvg_frag = nullptr, *wo_frag = nullptr, *wo_bfrag = nullptr, *dx_frag = nullptr;
   const h16* wqkvg = nullptr;   // [C][4HD]
   const h16* wo_t = nullptr;    // [C][HD]
   const h16* wo = nullptr;      // [HD][C]

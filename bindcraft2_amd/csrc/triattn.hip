@@ -42,6 +42,194 @@ struct TriAttnSave {
   }
 };
 
+// ---------------------------------------------------------------------------
+// The backward's end in one kernel (C = 128 or 64 channels, H = 4 bias heads):
+//   dy  = dqkvg . Wcat^T                       (K = 4C)
+//   din = dout + LN'(dy + sum_h dbias_h w2d_h)  (the input LayerNorm's backward)
+// with the bias gradient's per-chunk partials added here, in chunk order (the
+// sums of the attention backward's reduction, which is not launched).
+//
+// A workgroup owns 16 RT rows.  Everything it reads -- its rows of dqkvg, x and
+// dout, the partials -- is requested before the first wait, and the product
+// then waits on weight fragments alone (32 output columns a wave, four K steps
+// ahead, one contiguous 1 KB a fragment).  The 128 x 128 GEMM tile with this
+// epilogue (same sums, same order) walks K in eight steps of exposed loads
+// behind a prologue for the partials, in 32 workgroups at N = 64: 17 us there
+// and at N = 128, against 5 and 11 here.
+struct DxArgs {
+  const h16 *dqkvg, *W;  // [M][4C]; dx_frags
+  const float *x, *ln_g, *mean, *rstd, *dres, *dbias, *wb, *gmul;
+  float* out;
+  long M;
+  int nt, nch;  // nt: the transposed pair's rows when > 0; nch: partials [nch][H][M]
+};
+
+// Fragment (n32 * 4C/32 + ks) * 2 + jj, lane 16 g + c: column 32 n32 + 16 jj + c
+// of Wcat^T at k = 32 ks + 8 g + e.
+std::vector<h16> dx_frags(const std::vector<float>& cat, int C) {  // cat: [C][4C]
+  std::vector<h16> f((size_t)C * 4 * C);
+  size_t o = 0;
+  for (int n32 = 0; n32 < C / 32; ++n32)
+    for (int ks = 0; ks < 4 * C / 32; ++ks)
+      for (int jj = 0; jj < 2; ++jj)
+        for (int l = 0; l < 64; ++l)
+          for (int e = 0; e < 8; ++e)
+            f[o++] = (h16)cat[(size_t)(32 * n32 + 16 * jj + (l & 15)) * 4 * C + 32 * ks + 8 * (l >> 4) + e];
+  return f;
+}
+
+template <int C, int RT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 2 ? 4 : 3, 4))) void
+triattn_dx_kernel(DxArgs a) {
+  constexpr int H = 4, K = 4 * C, KS = K / 32, BM = 16 * RT, LDX = K + 8, LDT = C + 4;
+  constexpr int WC = C / 32, TI = RT * WC / 4;  // column waves, row tiles a wave
+  constexpr int GK = 4, NG = KS / GK;           // K steps a fragment group, groups
+  constexpr int LPR = C / 8, RPP = 256 / LPR, PASS = BM / RPP;
+  static_assert(RT * WC % 4 == 0 && BM % RPP == 0 && LDT * 4 <= LDX * 2, "tile split");
+  __shared__ __attribute__((aligned(16))) char smem[BM * LDX * 2];
+  __shared__ __attribute__((aligned(16))) float wbs[C * H], dbs[BM * H];
+  h16* xs = reinterpret_cast<h16*>(smem);
+  float* T = reinterpret_cast<float*>(smem);
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wc = w % WC, wr = w / WC;
+  const long M = a.M, m0 = (long)blockIdx.x * BM;
+  const int fr = tid / LPR, c0 = (tid % LPR) * 8;
+
+  // rows past M read row M - 1 and store nothing
+  constexpr int XP = BM * K / 8 / 256;
+  h16x8 av[XP];
+#pragma unroll
+  for (int p = 0; p < XP; ++p) {
+    const int it = tid + 256 * p;
+    av[p] = ld8(a.dqkvg + min(m0 + it / (K / 8), M - 1) * K + (it % (K / 8)) * 8);
+  }
+  float xv[PASS][8], dr[PASS][8], mu[PASS], rs[PASS];
+  long src[PASS];
+#pragma unroll
+  for (int p = 0; p < PASS; ++p) {
+    const long m = min(m0 + p * RPP + fr, M - 1);
+    src[p] = ln_src_row(m, a.nt) * C + c0;
+    ld_f8(a.x + src[p], xv[p]);
+    ld_f8(a.dres + src[p], dr[p]);
+    mu[p] = a.mean[m];
+    rs[p] = a.rstd[m];
+  }
+  for (int i = tid; i < C * H; i += 256) wbs[i] = a.wb[i];
+  if (tid < BM * H) {
+    // dbs[r][h]: the partials in chunk order, sixteen loads in flight
+    const int r = tid % BM, h = tid / BM;
+    const long cs = (long)H * M;
+    const float* p = a.dbias + (long)h * M + min(m0 + r, M - 1);
+    float s = 0.f;
+    int c = 0;
+    for (; c + 16 <= a.nch; c += 16) {
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = p[(c + u) * cs];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s += v[u];
+    }
+    for (; c + 4 <= a.nch; c += 4) {
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = p[(c + u) * cs];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s += v[u];
+    }
+    for (; c < a.nch; ++c) s += p[c * cs];
+    dbs[r * H + h] = s;
+  }
+  h16x8 bf[2][GK][2];
+  auto load_b = [&](int grp, h16x8 (&b)[GK][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < GK; ++k)
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj)
+        b[k][jj] = ld8(a.W + ((long)((wc * KS + grp * GK + k) * 2 + jj) * 64 + lane) * 8);
+  };
+  load_b(0, bf[0]);
+#pragma unroll
+  for (int p = 0; p < XP; ++p) {
+    const int it = tid + 256 * p;
+    st8(xs + it / (K / 8) * LDX + (it % (K / 8)) * 8, av[p]);
+  }
+  __syncthreads();
+
+  f32x4 acc[TI][2];
+#pragma unroll
+  for (int i = 0; i < TI; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int grp = 0; grp < NG; ++grp) {
+    if (grp + 1 < NG) load_b(grp + 1, bf[(grp + 1) & 1]);
+#pragma unroll
+    for (int k = 0; k < GK; ++k)
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        const h16x8 xf = ld8(xs + ((wr * TI + i) * 16 + l16) * LDX + (grp * GK + k) * 32 + 8 * g);
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) acc[i][jj] = mfma16x16x32(bf[grp & 1][k][jj], xf, acc[i][jj]);
+      }
+  }
+  __syncthreads();  // every wave is done with xs, which T overlays
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj)
+      *reinterpret_cast<f32x4*>(T + ((wr * TI + i) * 16 + l16) * LDT + 32 * wc + 16 * jj + 4 * g) = acc[i][jj];
+  float gm[8];
+  ld_f8(a.ln_g + c0, gm);
+  const float gs = *a.gmul;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) gm[e] *= gs;
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < PASS; ++p) {
+    const int r = p * RPP + fr;
+    if (m0 + r >= M) continue;  // a row's lanes leave together
+    float gv[8];
+    ld_f8(T + r * LDT + c0, gv);
+    float db[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) db[h] = dbs[r * H + h];
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) gv[e] += db[h] * wbs[(c0 + e) * H + h];
+    float sg = 0.f, sgx = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      xv[p][e] = (xv[p][e] - mu[p]) * rs[p];
+      gv[e] *= gm[e];
+      sg += gv[e];
+      sgx += gv[e] * xv[p][e];
+    }
+    sg = group_sum<LPR>(sg) * (1.f / C);
+    sgx = group_sum<LPR>(sgx) * (1.f / C);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dr[p][e] += rs[p] * (gv[e] - sg - xv[p][e] * sgx);
+    st_f8(a.out + src[p], dr[p]);
+  }
+}
+
+// C = 128: up to 144 rows a CU (N = 192: 21.6 us against the GEMM's 25.6); past
+// that both run at the memory's rate and the GEMM's loads, spread over its K
+// steps, keep it busier (N = 224 29 against 26, 512 150 against 142).
+bool triattn_dx_fits(int C, long M) { return C == 64 || M <= 144L * device_cus(); }
+
+void triattn_dx(hipStream_t st, int C, const DxArgs& a) {
+  auto go = [&](auto c, auto rt) {
+    constexpr int RT = decltype(rt)::value;
+    const long nwg = (a.M + 16 * RT - 1) / (16 * RT);
+    hipLaunchKernelGGL((triattn_dx_kernel<decltype(c)::value, RT>), dim3((unsigned)nwg), dim3(256), 0,
+                       st, a);
+  };
+  using std::integral_constant;
+  if (C == 128) go(integral_constant<int, 128>(), integral_constant<int, 2>());
+  // 64 rows beyond: N = 416 49 us against 55
+  else if (a.M > 144L * device_cus()) go(integral_constant<int, 64>(), integral_constant<int, 4>());
+  else go(integral_constant<int, 64>(), integral_constant<int, 2>());
+}
+
 }  // namespace
 
 TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
@@ -78,6 +266,7 @@ TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
       const std::vector<float> c = cat();  // [C][4HD]
       return proj_frags(4 * HD, C, 0, [&](int n, int k) { return c[(size_t)k * 4 * HD + n]; });
     });
+    w.dx_frag = ws.derived<h16>("triattn.dx_frag:" + P, [&] { return dx_frags(cat(), C); });
   }
   w.bqkvg = ws.derived<float>("triattn.bqkvg:" + P, [&] {
     std::vector<float> b((size_t)4 * HD, 0.f);
@@ -91,7 +280,7 @@ TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
   w.bo = ws.f32(P + "attention/output_b");
   if (rows) {
     w.wo_frag = ws.derived<h16>("triattn.wo_frag:" + P, [&] {
-      return proj_frags(C, HD, 0, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
+      return proj_frags(C, HD, C, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
     });
     w.wo_bfrag = ws.derived<h16>("triattn.wo_bfrag:" + P, [&] {
       return proj_frags(HD, C, 0, [&](int n, int k) { return ow.data[(size_t)n * C + k]; });
@@ -255,14 +444,14 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   need.take<h16>((size_t)M * 4 * HD);       // dqkvg
   need.take<float>((size_t)nch * H * M);     // dbias partials
   need.take<float>((size_t)H * M);           // dbias
-  need.take<float>((size_t)M * C);           // dxn
+  if (!w.dx_frag) need.take<float>((size_t)M * C);  // dxn
   ar.reset(st, need.off);
   b.dO = ar.take_n<h16>((size_t)M * HD);
   b.nDsum = ar.take_n<float>((size_t)H * M);
   b.dqkvg = ar.take_n<h16>((size_t)M * 4 * HD);
   b.dbias_part = ar.take_n<float>((size_t)nch * H * M);
   b.dbias = ar.take_n<float>((size_t)H * M);
-  float* dxn = ar.take_n<float>((size_t)M * C);
+  float* dxn = w.dx_frag ? nullptr : ar.take_n<float>((size_t)M * C);
 
   // d(og) = (tbl * dout) . Wo^T, the dropout scale applied as A is loaded;
   // the epilogue continues through the gate (dO, dG, Dsum)
@@ -299,17 +488,26 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   a.o = sv.o; a.og = nullptr; a.ldo = HD;
   a.lse = sv.lse;
   b.scale = 1.f / std::sqrt((float)w.D);
-  b.dbias_deferred = C == 128 && H == 4;  // the dX product's epilogue adds the partials
+  b.dbias_deferred = w.dx_frag != nullptr;  // the dX product's kernel adds the partials
   attn_bwd(st, b);
 
+  if (w.dx_frag && triattn_dx_fits(C, M)) {
+    DxArgs d{};
+    d.dqkvg = b.dqkvg; d.W = w.dx_frag; d.M = M; d.nt = per_column ? N : 0;
+    d.x = pair_in; d.ln_g = w.ln_g; d.mean = sv.mean; d.rstd = sv.rstd; d.dres = dout; d.out = din;
+    d.dbias = nch == 1 ? b.dbias : b.dbias_part; d.nch = nch;
+    d.wb = w.w2d; d.gmul = sc + 1;
+    KTimed kt(BC2N_TN(C, "triattn.gemm_dx_ln"), st);
+    triattn_dx(st, C, d);
+    return;
+  }
   GemmArgs g2;
   g2.M = (int)M; g2.N = C; g2.K = 4 * HD;
   g2.A = b.dqkvg; g2.a_sm = 4L * HD; g2.a_sk = 1;
   g2.B = w.wqkvg; g2.b_sn = 4L * HD; g2.b_sk = 1;
   if (C == 128 && H == 4) {
-    // the input LayerNorm's backward (with the pair-bias projection's term,
-    // its per-chunk partials added in the epilogue: attn_bwd launched no
-    // reduction) and the residual add in the epilogue
+    // the input LayerNorm's backward (with the pair-bias projection's term, its
+    // per-chunk partials added in the epilogue) and the residual add
     const float* dbp = nch == 1 ? b.dbias : b.dbias_part;
     gemm<128, 128>(st, g2,
                    EpiLnBwd<4>(pair_in, w.ln_g, sv.mean, sv.rstd, dout, din, M, per_column ? N : 0,

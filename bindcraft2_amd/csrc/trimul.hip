@@ -99,14 +99,14 @@ struct EpiTrimulOut : EpiRows {
     float bb[8], tt[8], r[8];
     h16x8 gv;
   };
-  __device__ __forceinline__ void load(long m, int n, Pre& p) const {
+  __device__ __forceinline__ void load(long m, int n, Pre& p, int) const {
     const long o = m * C + n;
     ld_f8(bo + n, p.bb);
     p.gv = ld8(gout + o);
     if (tbl) ld_f8(tbl + (long)((int)m % nt) * C + n, p.tt);
     ld_f8(in + o, p.r);
   }
-  __device__ __forceinline__ void row(long m, int n, const float (&v)[8], Pre& p) const {
+  __device__ __forceinline__ void row(long m, int n, const float (&v)[8], Pre& p, int) const {
     const long o = m * C + n;
     float ov[8], gv[8];
 #pragma unroll
@@ -124,8 +124,8 @@ struct EpiTrimulOut : EpiRows {
   }
   __device__ __forceinline__ void row(int, int m, int n, const float (&v)[8]) const {
     Pre p;
-    load(m, n, p);
-    row((long)m, n, v, p);
+    load(m, n, p, 4);
+    row((long)m, n, v, p, 4);
   }
 };
 
