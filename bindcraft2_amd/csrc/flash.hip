@@ -188,36 +188,48 @@ __device__ __forceinline__ RowHeadQb row_tile_order(int bid, int R, int H, int n
 }
 
 // ------------------------------------------------------------------ forward
-// Workgroup = (row r, head h, 64 queries); 4 waves x 16 queries; N = 32*NKB
-// > 256.  Keys are processed in chunks of 128 (4 blocks of 32) staged in one
-// LDS buffer; the next chunk's K and V are loaded into registers while the
-// current one computes, so the buffer is small (five workgroups fit a CU)
-// and the register budget leaves four waves per SIMD.  A lane keeps its
-// query's 32 scores of the chunk (8 keys of every block) in registers.
-// Per score: the pair bias is the score MFMA's accumulator, then one fma
-// (the key mask), half a max, a subtract, the exponent and half a convert;
-// the row sum of the probabilities comes from the P V product itself (one
-// more MFMA per block with an all-ones operand), summed over the same h16
-// probabilities the numerator uses.  Online softmax across chunks: the
-// output accumulator and the row sum are rescaled once per chunk.
-template <int D, int NKB, int QW>
-__global__ __launch_bounds__(64 * QW) void attn_fwd_kernel(AttnArgs a) {
+// Workgroup = (row r, head h, 128 queries); 4 waves x 32 queries (two 16-query
+// tiles); N = 32*NKB > 256.  Keys are processed in chunks of 32 CB staged in
+// one of two LDS buffers, the next chunk's K and V loaded into registers while
+// the current one computes; one barrier a chunk.  A lane keeps its two queries'
+// scores of the chunk (8 keys of every block each) in registers.
+//
+// No one unit bounds it: at N = 512 the bias reads from L2 (1 GB a launch) take
+// 30 us of 206, K and V's 15, the exponentials 14 (variants without each), about
+// 70 are HBM's, and LDS reads and the other per-score instructions add to them:
+//  * With 16 queries a wave every 32 keys cost K, V and two mask vectors, 64 LDS
+//    cycles for 512 scores; two query tiles share the K, V and mask reads, and
+//    the mask is one vector: 48 cycles for 1024.
+//  * Per score: one v_fma_mix_f32 makes the score MFMA's accumulator from the
+//    binary16 bias and the additive mask, then half a max, a subtract, the
+//    exponent and half a convert; the row sum of the probabilities comes from
+//    the P V product itself (one more MFMA per block with an all-ones operand),
+//    summed over the same h16 probabilities the numerator uses.
+//  * 64 keys a chunk (113 registers: four waves a SIMD); 96 from N = 480.
+// N = 288 / 416 / 512: 54 / 140 / 218 us a launch with 16 queries a wave, 50 /
+// 124 / 205 so.  Two rows a workgroup, the bias shared in registers, leave three
+// waves a SIMD and are slower (71 / 169 / 222), and so are 5 to 7 waves (56 / 131
+// / 209): too few workgroups a CU.
+// A masked key's score is NEG_LOGIT plus its unmasked score: weight exactly 0
+// beside any live key.  In a fully masked row the bias factor `br` and q are 0,
+// so every key scores exactly NEG_LOGIT and the row attends uniformly.
+// Online softmax across chunks: the output accumulator and the row sum are
+// rescaled once per chunk.
+template <int D, int NKB, int CB>
+__global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   constexpr int DT = D / 16;
   constexpr int LD = lds_ld<D>();
   constexpr int N = 32 * NKB;  // == a.N (dispatch)
-  constexpr int CB = 4;        // key blocks per chunk
+  constexpr int QT = 2, QW = 4, T = 64 * QW, QR = 16 * QT * QW;  // queries a workgroup
   constexpr int CN = 32 * CB;  // keys per chunk
   constexpr int NFULL = NKB / CB, TAIL = NKB % CB;
   constexpr int NCH = NFULL + (TAIL ? 1 : 0);
   const int H = a.H;
-  h16* Ks = reinterpret_cast<h16*>(smem_raw);          // [CN][LD]
-  h16* Vs = Ks + CN * LD;                               // [CN][LD]
-  float* Mm = reinterpret_cast<float*>(Vs + CN * LD);    // [N] 1 / 0 per key
-  float* Ma = Mm + N;                                    // [N] 0 / NEG_LOGIT
-  constexpr int T = 64 * QW;   // threads; QW waves of 16 queries
+  h16* KV = reinterpret_cast<h16*>(smem_raw);            // [2][K, V][CN][LD]
+  float* Ma = reinterpret_cast<float*>(KV + 4 * CN * LD);  // [N] 0 / NEG_LOGIT
 
-  const int nqb = (N + 16 * QW - 1) / (16 * QW);
+  constexpr int nqb = (N + QR - 1) / QR;
   const long G = (long)a.R * H * nqb;
   const int bid = (int)xcd_block(G);
   if (bid >= G) return;
@@ -230,126 +242,158 @@ __global__ __launch_bounds__(64 * QW) void attn_fwd_kernel(AttnArgs a) {
   const h16* Vg = a.qkvg + tok0 * a.ld + 2 * H * D + h * D;
   RowPair<D, CN, T> nkv;  // the next chunk's K and V rows
   nkv.load(Kg, a.ld, Vg, a.ld, tid, min(CN, N));
+  int on = 0;
   for (int k = tid; k < N; k += T) {
-    const bool on = a.mask[r * a.mask_sr + k * a.mask_sk] != 0.f;
-    Mm[k] = on ? 1.f : 0.f;
-    Ma[k] = on ? 0.f : NEG_LOGIT;
+    const bool o = a.mask[r * a.mask_sr + k * a.mask_sk] != 0.f;
+    on |= o;
+    Ma[k] = o ? 0.f : NEG_LOGIT;
   }
 
-  const int q0 = qb * 16 * QW + wave * 16;
-  const bool active = q0 < N;  // idle waves keep to the barriers only
+  const int q0 = qb * QR + wave * 16 * QT;
+  const bool active = q0 < N;  // idle waves keep to the barriers only (N % 32 == 0: whole waves)
   const int lq = lane & 15, g = lane >> 4;
-  const int q = min(q0, N - 16) + lq;  // idle waves read in bounds, store nothing
-  HFrag<D> qf;
-  qf.load(a.qkvg + (tok0 + q) * a.ld + h * D, g);
-  const h16* grow = a.qkvg + (tok0 + q) * a.ld + 3 * H * D + h * D;
-  h16x4 gv[DT];
+  const int qw = min(q0, N - 16 * QT);  // idle waves read in bounds, store nothing
+  HFrag<D> qf[QT];
 #pragma unroll
-  for (int dh = 0; dh < DT; ++dh) gv[dh] = *reinterpret_cast<const h16x4*>(grow + dh * 16 + 4 * g);
-  const int qt = q >> 4;  // the wave's 16-query tile (bias blocks; the launcher requires the bias)
+  for (int t = 0; t < QT; ++t) qf[t].load(a.qkvg + (tok0 + qw + 16 * t + lq) * a.ld + h * D, g);
+  const bool live = __syncthreads_or(on);  // the row has an unmasked key
+  float br = live ? 1.f : 0.f;
+  asm volatile("" : "+v"(br));  // a register operand: with a literal 1 the fma becomes two instructions
+  if (!live) {
+#pragma unroll
+    for (int t = 0; t < QT; ++t) qf[t].v = {};
+  }
   const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
   h16x8 ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (h16)1.f;
-  float mx = -INFINITY;  // running maximum (exp2(-inf - m) = 0 rescales nothing)
-  f32x4 acc[DT], lacc = z4;
+  float mx[QT];  // running maximum (exp2(-inf - m) = 0 rescales nothing)
+  f32x4 acc[QT][DT], lacc[QT];
 #pragma unroll
-  for (int i = 0; i < DT; ++i) acc[i] = z4;
+  for (int t = 0; t < QT; ++t) {
+    mx[t] = -INFINITY;
+    lacc[t] = z4;
+#pragma unroll
+    for (int i = 0; i < DT; ++i) acc[t][i] = z4;
+  }
+  nkv.store(KV, KV + CN * LD, tid, min(CN, N));
+  if (NCH > 1)
+    nkv.load(Kg + (long)CN * a.ld, a.ld, Vg + (long)CN * a.ld, a.ld, tid, min(CN, N - CN));
+  __syncthreads();
 
-  auto chunk = [&](int c, auto nbc) {
+  auto chunk = [&](int c, auto nbc) __attribute__((always_inline)) {
     constexpr int NBC = decltype(nbc)::value;  // key blocks in this chunk
     const int k0 = c * CN;
-    // the chunk's pair bias: the score MFMAs' accumulators
-    f32x4 sv[NBC][2];
-#pragma unroll
-    for (int kb = 0; kb < NBC; ++kb) {
-      const h16x8 bb = ld8(bias_frag_block(a.bias, h, qt, (k0 >> 5) + kb, N, lane));
-#pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sv[kb][kh][i] = (float)bb[kh * 4 + i];
-    }
-    __syncthreads();  // the previous chunk's LDS readers are done
-    nkv.store(Ks, Vs, tid, NBC * 32);
-    __syncthreads();
-    // the next chunk's K and V, issued after this chunk's scores (the wait
-    // counter retires loads in order: issued earlier, they would hold up
-    // the scores' wait for the bias)
-    auto prefetch = [&] {
-      if (c + 1 < NCH)
-        nkv.load(Kg + (long)(k0 + CN) * a.ld, a.ld, Vg + (long)(k0 + CN) * a.ld, a.ld, tid,
-                 min(CN, N - k0 - CN));
-    };
-    float mc = -INFINITY;
+    const h16* Ks = KV + (c & 1) * 2 * CN * LD;
+    const h16* Vs = Ks + CN * LD;
     if (active) {
+      h16x8 bb[NBC][QT];
 #pragma unroll
-      for (int kb = 0; kb < NBC; ++kb) {
+      for (int kb = 0; kb < NBC; ++kb)
+#pragma unroll
+        for (int t = 0; t < QT; ++t)
+          bb[kb][t] = ld8(bias_frag_block(a.bias, h, (qw >> 4) + t, (k0 >> 5) + kb, N, lane));
+      f32x4 sv[NBC][2][QT];
+      float mc[QT];
+#pragma unroll
+      for (int t = 0; t < QT; ++t) mc[t] = -INFINITY;
+#pragma unroll
+      for (int kb = 0; kb < NBC; ++kb)
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh) {
           HFrag<D> kf;
           kf.load(&Ks[(kb * 32 + kh * 16 + lq) * LD], g);
-          sv[kb][kh] = HFrag<D>::mma(kf, qf, sv[kb][kh]);  // score + bias
-          const int kk = k0 + kb * 32 + kh * 16 + 4 * g;
-          const float4 mm = *reinterpret_cast<const float4*>(Mm + kk);
-          const float4 ma = *reinterpret_cast<const float4*>(Ma + kk);
-          const float mv[4] = {mm.x, mm.y, mm.z, mm.w};
-          const float av[4] = {ma.x, ma.y, ma.z, ma.w};
+          const float4 m4 = *reinterpret_cast<const float4*>(Ma + k0 + kb * 32 + kh * 16 + 4 * g);
+          const float ma[4] = {m4.x, m4.y, m4.z, m4.w};
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            // unmasked: s + bias; masked: exactly NEG_LOGIT
-            const float x = __builtin_fmaf(sv[kb][kh][i], mv[i], av[i]);
-            sv[kb][kh][i] = x;
-            mc = fmaxf(mc, x);
+          for (int t = 0; t < QT; ++t) {
+            f32x4 cs;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              cs[i] = __builtin_fmaf((float)bb[kb][t][kh * 4 + i], br, ma[i]);
+            sv[kb][kh][t] = HFrag<D>::mma(kf, qf[t], cs);  // score + bias + mask
           }
         }
+#pragma unroll
+      for (int kb = 0; kb < NBC; ++kb)
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+          for (int t = 0; t < QT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mc[t] = fmaxf(mc[t], sv[kb][kh][t][i]);
+#pragma unroll
+      for (int t = 0; t < QT; ++t) {
+        mc[t] = fmaxf(mc[t], __shfl_xor(mc[t], 16, 64));
+        mc[t] = fmaxf(mc[t], __shfl_xor(mc[t], 32, 64));
+        const float mn = fmaxf(mx[t], mc[t]);
+        const float alpha = fast_exp2(mx[t] - mn);
+#pragma unroll
+        for (int dh = 0; dh < DT; ++dh) acc[t][dh] *= alpha;
+        lacc[t] *= alpha;
+        mx[t] = mn;
+      }
+#pragma unroll
+      for (int kb = 0; kb < NBC; ++kb) {
+        h16x8 pf[QT];
+#pragma unroll
+        for (int t = 0; t < QT; ++t)
+#pragma unroll
+          for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              pf[t][kh * 4 + i] = (h16)fast_exp2(sv[kb][kh][t][i] - mx[t]);
+#pragma unroll
+        for (int dh = 0; dh < DT; ++dh) {
+          const h16x8 vf = ld_tr8(Vs, LD, kb * 32, dh * 16, lane);
+#pragma unroll
+          for (int t = 0; t < QT; ++t) acc[t][dh] = mfma16x16x32(vf, pf[t], acc[t][dh]);
+        }
+#pragma unroll
+        for (int t = 0; t < QT; ++t) lacc[t] = mfma16x16x32(ones, pf[t], lacc[t]);
       }
     }
-    prefetch();
-    if (!active) return;
-    mc = fmaxf(mc, __shfl_xor(mc, 16, 64));
-    mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
-    const float mn = fmaxf(mx, mc);
-    const float alpha = fast_exp2(mx - mn);
-#pragma unroll
-    for (int dh = 0; dh < DT; ++dh) acc[dh] *= alpha;
-    lacc *= alpha;
-    mx = mn;
-#pragma unroll
-    for (int kb = 0; kb < NBC; ++kb) {
-      h16x8 pf;
-#pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pf[kh * 4 + i] = (h16)fast_exp2(sv[kb][kh][i] - mx);
-#pragma unroll
-      for (int dh = 0; dh < DT; ++dh)
-        acc[dh] = mfma16x16x32(ld_tr8(Vs, LD, kb * 32, dh * 16, lane), pf, acc[dh]);
-      lacc = mfma16x16x32(ones, pf, lacc);  // row sum of the probabilities
+    if (c + 1 < NCH) {
+      // the other buffer's readers finished before the last barrier
+      h16* Kn = KV + ((c + 1) & 1) * 2 * CN * LD;
+      nkv.store(Kn, Kn + CN * LD, tid, min(CN, N - k0 - CN));
+      if (c + 2 < NCH)
+        nkv.load(Kg + (long)(k0 + 2 * CN) * a.ld, a.ld, Vg + (long)(k0 + 2 * CN) * a.ld, a.ld, tid,
+                 min(CN, N - k0 - 2 * CN));
+      __syncthreads();
     }
   };
-  // unrolled, so the wait for each chunk's loads counts only what is in flight
-#pragma unroll
+  // 64-key chunks in a loop (unrolled, later chunks' loads take registers: N =
+  // 416 129 us against 124, 448 160 / 154), 96-key ones unrolled (N = 512 205 / 210)
+  constexpr int UNROLL = CB == 2 ? 1 : NFULL;
+#pragma unroll UNROLL
   for (int c = 0; c < NFULL; ++c) chunk(c, std::integral_constant<int, CB>());
   if constexpr (TAIL > 0) chunk(NFULL, std::integral_constant<int, TAIL>());
 
   if (!active) return;
-  const float lsum = lacc[0];
-  const float inv = __builtin_amdgcn_rcpf(lsum);
-  const long orow = (tok0 + q) * a.ldo + h * D;
 #pragma unroll
-  for (int dh = 0; dh < DT; ++dh) {
-    const int d0 = dh * 16 + 4 * g;
-    h16x4 ov, gov;
+  for (int t = 0; t < QT; ++t) {
+    const int q = qw + 16 * t + lq;
+    const h16* grow = a.qkvg + (tok0 + q) * a.ld + 3 * H * D + h * D;
+    const float lsum = lacc[t][0];
+    const float inv = __builtin_amdgcn_rcpf(lsum);
+    const long orow = (tok0 + q) * a.ldo + h * D;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float o = acc[dh][i] * inv;
-      ov[i] = (h16)o;
-      gov[i] = (h16)(o * sigmoidf_((float)gv[dh][i]));
+    for (int dh = 0; dh < DT; ++dh) {
+      const int d0 = dh * 16 + 4 * g;
+      const h16x4 gv = *reinterpret_cast<const h16x4*>(grow + d0);
+      h16x4 ov, gov;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float o = acc[t][dh][i] * inv;
+        ov[i] = (h16)o;
+        gov[i] = (h16)(o * sigmoidf_((float)gv[i]));
+      }
+      *reinterpret_cast<h16x4*>(a.o + orow + d0) = ov;
+      *reinterpret_cast<h16x4*>(a.og + orow + d0) = gov;
     }
-    *reinterpret_cast<h16x4*>(a.o + orow + d0) = ov;
-    *reinterpret_cast<h16x4*>(a.og + orow + d0) = gov;
+    if (g == 0) a.lse[((long)r * H + h) * N + q] = mx[t] + __log2f(lsum);
   }
-  if (g == 0) a.lse[((long)r * H + h) * N + q] = mx + __log2f(lsum);
 }
 
 // Forward over a chunk of rows, N <= 256 (one key chunk).  Workgroup = (row
@@ -560,27 +604,29 @@ __global__ __launch_bounds__(256) void attn_gate_bwd_kernel(AttnBwdArgs b) {
 }
 
 // ----------------------------------------------------------- backward: dQ
-// Same decomposition as the forward: (row, head, 64 queries), 4 waves, keys
-// in chunks of up to 256 staged in LDS.  Per chunk the lane's pair-bias row
-// (minus lse, with -inf at masked keys so p = dS = 0 there) is fetched up
-// front, all loads in flight at once.
-template <int D, int NKB, int QW>
-__global__ __launch_bounds__(64 * QW) void attn_bwd_dq_kernel(AttnBwdArgs b) {
+// The forward's decomposition beyond N = 256: (row, head, 128 queries), 4 waves
+// x 32 queries, keys in chunks of 32 CB through two LDS buffers.  The score
+// MFMA starts from bias - lse (one v_fma_mix_f32 from the binary16 bias) plus
+// the mask, -inf at masked keys so p = dS = 0 there; dP's from -Dsum.  K, V,
+// mask and transposed K reads, 64 LDS cycles a 32-key block, serve two query
+// tiles.  N = 288 / 416 / 512: 51 / 135 / 198 us a
+// launch with 16 queries a wave and 256 keys a chunk, 43 / 113 / 178 so.
+template <int D, int NKB, int CB>
+__global__ __launch_bounds__(256) void attn_bwd_dq_kernel(AttnBwdArgs b) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   constexpr int DT = D / 16;
   constexpr int LD = lds_ld<D>();
   const AttnArgs& a = b.f;
   constexpr int N = 32 * NKB;  // == a.N (dispatch)
-  constexpr int CB = NKB < 8 ? NKB : 8;  // key blocks per chunk
-  constexpr int NCH = (NKB + CB - 1) / CB;
-  constexpr int CN = 32 * CB;
+  constexpr int QT = 2, QW = 4, T = 64 * QW, QR = 16 * QT * QW;  // queries a workgroup
+  constexpr int CN = 32 * CB;  // keys per chunk
+  constexpr int NFULL = NKB / CB, TAIL = NKB % CB;
+  constexpr int NCH = NFULL + (TAIL ? 1 : 0);
   const int H = a.H;
-  h16* Ks = reinterpret_cast<h16*>(smem_raw);   // [CN][LD]
-  h16* Vs = Ks + CN * LD;                        // [CN][LD]
-  float* Ms = reinterpret_cast<float*>(Vs + CN * LD);  // [N]
-  constexpr int T = 64 * QW;   // threads; QW waves of 16 queries
+  h16* KV = reinterpret_cast<h16*>(smem_raw);             // [2][K, V][CN][LD]
+  float* Ms = reinterpret_cast<float*>(KV + 4 * CN * LD);  // [N] 0 / -inf
 
-  const int nqb = (N + 16 * QW - 1) / (16 * QW);
+  constexpr int nqb = (N + QR - 1) / QR;
   const long G = (long)a.R * H * nqb;
   const int bid = (int)xcd_block(G);
   if (bid >= G) return;
@@ -591,89 +637,107 @@ __global__ __launch_bounds__(64 * QW) void attn_bwd_dq_kernel(AttnBwdArgs b) {
   const long tok0 = (long)r * N;
   const h16* Kg = a.qkvg + tok0 * a.ld + H * D + h * D;
   const h16* Vg = a.qkvg + tok0 * a.ld + 2 * H * D + h * D;
-  stage_rows2<D, CN, T>(Ks, Kg, a.ld, Vs, Vg, a.ld, tid);
-  // additive key mask: a masked key's exponent becomes -inf, so p = dS = 0
+  RowPair<D, CN, T> nkv;  // the next chunk's K and V rows
+  nkv.load(Kg, a.ld, Vg, a.ld, tid, min(CN, N));
   for (int k = tid; k < N; k += T)
     Ms[k] = a.mask[r * a.mask_sr + k * a.mask_sk] != 0.f ? 0.f : -INFINITY;
 
-  const int q0 = qb * 16 * QW + wave * 16;
+  const int q0 = qb * QR + wave * 16 * QT;
+  const bool active = q0 < N;  // idle waves keep to the barriers only (N % 32 == 0: whole waves)
   const int lq = lane & 15, g = lane >> 4;
-  const int q = min(q0, N - 16) + lq;  // idle waves read in bounds, store nothing
-  HFrag<D> qf, dof;
-  qf.load(a.qkvg + (tok0 + q) * a.ld + h * D, g);
-  dof.load(b.dO + (tok0 + q) * a.ldo + h * D, g);
-  const float lse = a.lse[((long)r * H + h) * N + q];
-  const float nDq = b.nDsum[((long)r * H + h) * N + q];
-  const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
-  const f32x4 nD = {nDq, nDq, nDq, nDq};
-  f32x4 acc[DT];
+  const int qw = min(q0, N - 16 * QT);  // idle waves read in bounds, store nothing
+  HFrag<D> qf[QT], dof[QT];
+  float lse[QT];
+  f32x4 nD[QT], acc[QT][DT];
 #pragma unroll
-  for (int i = 0; i < DT; ++i) acc[i] = z4;
+  for (int t = 0; t < QT; ++t) {
+    const int q = qw + 16 * t + lq;
+    qf[t].load(a.qkvg + (tok0 + q) * a.ld + h * D, g);
+    dof[t].load(b.dO + (tok0 + q) * a.ldo + h * D, g);
+    lse[t] = a.lse[((long)r * H + h) * N + q];
+    const float d = b.nDsum[((long)r * H + h) * N + q];
+    nD[t] = f32x4{d, d, d, d};
+#pragma unroll
+    for (int i = 0; i < DT; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float one = 1.f;
+  asm volatile("" : "+v"(one));  // a register operand: with a literal 1 the fma becomes two instructions
+  nkv.store(KV, KV + CN * LD, tid, min(CN, N));
+  if (NCH > 1)
+    nkv.load(Kg + (long)CN * a.ld, a.ld, Vg + (long)CN * a.ld, a.ld, tid, min(CN, N - CN));
+  __syncthreads();
 
+  auto chunk = [&](int c, auto nbc) __attribute__((always_inline)) {
+    constexpr int NBC = decltype(nbc)::value;  // key blocks in this chunk
+    const int k0 = c * CN;
+    const h16* Ks = KV + (c & 1) * 2 * CN * LD;
+    const h16* Vs = Ks + CN * LD;
+    if (active) {
+      h16x8 bb[NBC][QT];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    const int k0c = c * CN;
-    float bsv[CB][8];
+      for (int kb = 0; kb < NBC; ++kb)
 #pragma unroll
-    for (int kb = 0; kb < CB; ++kb) {
-      if (c * CB + kb < NKB) {
-        const h16x8 bb = ld8(bias_frag_block(a.bias, h, q >> 4, (k0c >> 5) + kb, N, lane));
+        for (int t = 0; t < QT; ++t)
+          bb[kb][t] = ld8(bias_frag_block(a.bias, h, (qw >> 4) + t, (k0 >> 5) + kb, N, lane));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) bsv[kb][e] = (float)bb[e] - lse;
-      }
-    }
-    if (c > 0) {
-      __syncthreads();  // every wave is done with the previous chunk
-      stage_rows2<D, CN, T>(Ks, Kg + (long)k0c * a.ld, a.ld, Vs, Vg + (long)k0c * a.ld, a.ld, tid,
-                            min(CN, N - k0c));
-    }
-    __syncthreads();
-    if (NCH == 1 && q0 >= N) return;  // idle wave, no barrier follows
-#pragma unroll
-    for (int kb = 0; kb < CB; ++kb) {
-      if (c * CB + kb < NKB) {
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
-          const float4 mm = *reinterpret_cast<const float4*>(Ms + k0c + kb * 32 + kh * 16 + 4 * g);
-          bsv[kb][kh * 4 + 0] += mm.x;
-          bsv[kb][kh * 4 + 1] += mm.y;
-          bsv[kb][kh * 4 + 2] += mm.z;
-          bsv[kb][kh * 4 + 3] += mm.w;
-        }
-      }
-    }
-#pragma unroll
-    for (int kb = 0; kb < CB; ++kb) {
-      if (c * CB + kb < NKB) {
-        h16x8 dsf;
+      for (int kb = 0; kb < NBC; ++kb) {
+        h16x8 dsf[QT];
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh) {
           const int krow = (kb * 32 + kh * 16 + lq) * LD;
           HFrag<D> kf, vf;
           kf.load(&Ks[krow], g);
           vf.load(&Vs[krow], g);
-          f32x4 cs;
+          const float4 m4 = *reinterpret_cast<const float4*>(Ms + k0 + kb * 32 + kh * 16 + 4 * g);
+          const float ms[4] = {m4.x, m4.y, m4.z, m4.w};
+          f32x4 s[QT], dp[QT];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) cs[i] = bsv[kb][kh * 4 + i];
-          const f32x4 s = HFrag<D>::mma(kf, qf, cs);    // S + bias - lse
-          const f32x4 dp = HFrag<D>::mma(vf, dof, nD);  // dP - Dsum
+          for (int t = 0; t < QT; ++t) {
+            f32x4 cs;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) dsf[kh * 4 + i] = (h16)(fast_exp2(s[i]) * dp[i]);
+            for (int i = 0; i < 4; ++i)
+              cs[i] = __builtin_fmaf((float)bb[kb][t][kh * 4 + i], one, -lse[t]) + ms[i];
+            s[t] = HFrag<D>::mma(kf, qf[t], cs);      // S + bias - lse
+            dp[t] = HFrag<D>::mma(vf, dof[t], nD[t]);  // dP - Dsum
+          }
+#pragma unroll
+          for (int t = 0; t < QT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dsf[t][kh * 4 + i] = (h16)(fast_exp2(s[t][i]) * dp[t][i]);
         }
 #pragma unroll
-        for (int dh = 0; dh < DT; ++dh)
-          acc[dh] = mfma16x16x32(ld_tr8(Ks, LD, kb * 32, dh * 16, lane), dsf, acc[dh]);
+        for (int dh = 0; dh < DT; ++dh) {
+          const h16x8 kt = ld_tr8(Ks, LD, kb * 32, dh * 16, lane);
+#pragma unroll
+          for (int t = 0; t < QT; ++t) acc[t][dh] = mfma16x16x32(kt, dsf[t], acc[t][dh]);
+        }
       }
     }
-  }
-  if (q0 >= N) return;
-  h16* out = b.dqkvg + (tok0 + q) * a.ld + h * D;
+    if (c + 1 < NCH) {
+      // the other buffer's readers finished before the last barrier
+      h16* Kn = KV + ((c + 1) & 1) * 2 * CN * LD;
+      nkv.store(Kn, Kn + CN * LD, tid, min(CN, N - k0 - CN));
+      if (c + 2 < NCH)
+        nkv.load(Kg + (long)(k0 + 2 * CN) * a.ld, a.ld, Vg + (long)(k0 + 2 * CN) * a.ld, a.ld, tid,
+                 min(CN, N - k0 - 2 * CN));
+      __syncthreads();
+    }
+  };
 #pragma unroll
-  for (int dh = 0; dh < DT; ++dh) {
-    h16x4 v;
+  for (int c = 0; c < NFULL; ++c) chunk(c, std::integral_constant<int, CB>());
+  if constexpr (TAIL > 0) chunk(NFULL, std::integral_constant<int, TAIL>());
+
+  if (!active) return;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = (h16)(acc[dh][i] * b.scale);
-    *reinterpret_cast<h16x4*>(out + dh * 16 + 4 * g) = v;
+  for (int t = 0; t < QT; ++t) {
+    h16* out = b.dqkvg + (tok0 + qw + 16 * t + lq) * a.ld + h * D;
+#pragma unroll
+    for (int dh = 0; dh < DT; ++dh) {
+      h16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (h16)(acc[t][dh][i] * b.scale);
+      *reinterpret_cast<h16x4*>(out + dh * 16 + 4 * g) = v;
+    }
   }
 }
 
@@ -1165,6 +1229,17 @@ __device__ __forceinline__ void wait_vm() {
 //    count, each takes one 16-query half of the last block.
 //  * Two barriers per row: one after the copies land, one to add the query
 //    groups' dK/dV partials.
+//  * Two workgroups share a CU's 160 KB of LDS: two row buffers and 8 KB of
+//    partials each up to N = 224 (79 KB), and at N = 256, where that would be
+//    88, the partials go over the row's own buffer, for one more barrier a row
+//    (one workgroup a CU there made its one round of workgroups two: 71.5 us a
+//    launch against 48.9).
+constexpr int dkv_row_bytes(int N) { return 2 * N * 64 + 2 * 32 * 64 + 3 * N * 4; }
+constexpr int DKV_X_BYTES = 2 * 2 * 8 * 64 * 4;  // [key tile][K, V][8][64] f32, query group 1
+constexpr bool dkv_x_over(int N) { return 2 * (2 * dkv_row_bytes(N) + DKV_X_BYTES) > 160 * 1024; }
+constexpr int dkv_lds_bytes(int N) {
+  return 2 * dkv_row_bytes(N) + (dkv_x_over(N) ? 0 : DKV_X_BYTES);
+}
 template <int NQB>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_lds_kernel(AttnBwdArgs b) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -1179,13 +1254,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_lds_kernel(AttnBwdArgs b)
   constexpr int KVT = 16 * KT * 64;      // bytes of the K (or V) tile
   constexpr int SOFF = 2 * TILE + 2 * KVT;
   constexpr int BUF = SOFF + 3 * N * 4;
+  static_assert(BUF == dkv_row_bytes(N), "row buffer");
+  constexpr bool XOVER = dkv_x_over(N);
   constexpr int JT = N / 16;             // 1 KB copies per Q (dO) tile
   constexpr int NCP = NQB + 1;           // tile copies per wave: (2 JT + 2 KT) / 4
   constexpr int JS = (N + 63) / 64;      // 256-byte copies per statistic
   constexpr int NSC = (3 * JS + 3) / 4;  // statistic copies per wave (at most)
   const AttnArgs& a = b.f;
   const int H = a.H;
-  float* Xs = reinterpret_cast<float*>(smem_raw + 2 * BUF);  // [KT][K,V][DT*4][64], query group 1
 
   constexpr int NKW = N / (16 * KT);
   const long G = (long)((a.R + b.rows_per_chunk - 1) / b.rows_per_chunk) * H * NKW;
@@ -1412,6 +1488,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_lds_kernel(AttnBwdArgs b)
 
     // row done: query group 1 parks its partials, query group 0 adds them
     // and writes dK, dV of its key tile
+    float* Xs = reinterpret_cast<float*>(smem_raw + (XOVER ? u : 2) * BUF);
+    if constexpr (XOVER) __syncthreads();  // every wave is done with the row's buffer
     if (qs == 1) {
       float* x = Xs + kt_ * (2 * DT * 4 * 64);
 #pragma unroll
@@ -1920,15 +1998,14 @@ static void attn_fwd_t(hipStream_t st, const AttnArgs& a) {
     return;
   }
   if (!a.bias) throw std::runtime_error("attention: the chunked forward needs the pair bias");
-  // one 128-key K/V buffer + the row's key mask (two floats a key); eight
-  // waves (128 queries) a workgroup, so each row's K/V is read by N / 128
-  // workgroups
-  constexpr int QW = 8;
-  const size_t lds = (size_t)128 * lds_ld<D>() * 2 * 2 + (size_t)a.N * 8;
-  const dim3 grid(xcd_grid((long)a.R * a.H * ((a.N + 16 * QW - 1) / (16 * QW))));
+  const dim3 grid(xcd_grid((long)a.R * a.H * ((a.N + 127) / 128)));
   with_blocks(a.N / 32, [&](auto nb) {
-    hipLaunchKernelGGL((attn_fwd_kernel<D, decltype(nb)::value, QW>), grid, dim3(64 * QW), lds, st,
-                       a);
+    constexpr int NB = decltype(nb)::value, CB = NB >= 15 ? 3 : 2;  // key blocks a chunk
+    if constexpr (NB > 8) {
+      // two K/V buffers and the key mask
+      const size_t lds = (size_t)4 * 32 * CB * lds_ld<D>() * 2 + (size_t)a.N * 4;
+      hipLaunchKernelGGL((attn_fwd_kernel<D, NB, CB>), grid, dim3(256), lds, st, a);
+    }
   });
 }
 
@@ -1969,13 +2046,14 @@ static void attn_bwd_t(hipStream_t st, const AttnBwdArgs& b0) {
     });
   } else {
     if (!a.bias) throw std::runtime_error("attention: the chunked dQ needs the pair bias");
-    const size_t lds_q = (size_t)attn_chunk(a.N) * lds_ld<D>() * 2 * 2 + (size_t)a.N * 4;
     KTimed kt(timer_name(2, a), st);
-    constexpr int QW = 8;  // 128 queries a workgroup, as the forward
-    const dim3 grid(xcd_grid((long)a.R * a.H * ((a.N + 16 * QW - 1) / (16 * QW))));
+    const dim3 grid(xcd_grid((long)a.R * a.H * ((a.N + 127) / 128)));  // as the forward
     with_blocks(a.N / 32, [&](auto nb) {
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, decltype(nb)::value, QW>), grid, dim3(64 * QW),
-                         lds_q, st, b);
+      constexpr int NB = decltype(nb)::value, CB = 2;  // key blocks a chunk
+      if constexpr (NB > 8) {
+        const size_t lds = (size_t)4 * 32 * CB * lds_ld<D>() * 2 + (size_t)a.N * 4;
+        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NB, CB>), grid, dim3(256), lds, st, b);
+      }
     });
   }
   const int nch = attn_bwd_nchunk(a.R, b.rows_per_chunk);
@@ -1991,8 +2069,7 @@ static void attn_bwd_t(hipStream_t st, const AttnBwdArgs& b0) {
     const dim3 grid(xcd_grid((long)nch * a.H * nkw));
     if constexpr (D == 32) {
       if (a.N <= 256 && a.bias) {
-        // two row buffers (Q, dO tiles + lse, -Dsum, mask) + 4 waves' partials
-        const size_t lds = (size_t)2 * (2 * a.N * 64 + 3 * a.N * 4) + (size_t)4 * 2 * 2 * 4 * 64 * 4;
+        const size_t lds = dkv_lds_bytes(a.N);
         with_blocks(a.N / 32, [&](auto nb) {
           if constexpr (decltype(nb)::value <= 8)
             hipLaunchKernelGGL((attn_bwd_dkv_lds_kernel<decltype(nb)::value>), grid, dim3(256), lds,
