@@ -313,34 +313,36 @@ void block_bwd(hipStream_t st, const BlockW& B, const Layout& L, int b, const Ta
       KTimed kt("block.ct_scale", ms);
       ct_scale(ms, dmsa, (long)S * N * L.Cm, sm);
     }
-    transition_bwd(ms, B.mtr, (long)S * N, N, p.m2, nullptr, p.mtr, dmsa, dmsa, sm);
+    transition_bwd(ms, B.mtr, (long)S * N, N, p.m2, nullptr, p.mtr, dmsa, dmsa, CtScale{sm});
     msacol_bwd(ms, B.col, S, N, p.m1, mmask, nullptr, p.col, dmsa, dmsa, sm);
     dbias = msarow_bwd_msa(ms, B.row, S, N, f.min, mmask, t.row(b), p.row, dmsa, dmsa, sm);
   }
   // the pair scale alternates two slots a block when the OPM backward that
   // reads it is deferred past the next block's ct_scale
+  // (its final reduction is left to the transition's kernel where that reduces it)
   float* sp = ct_scale_slot(two ? 4 + (b & 1) : 1);
+  CtScale spl;
   {
     KTimed kt("block.ct_scale", st);
     if (pipe && pipe->amax_np > 0 && pipe->amax_of == dp_in)
-      ct_scale_parts(st, ct_fused_parts(), pipe->amax_np, sp);
+      spl = ct_scale_parts_lazy(st, ct_fused_parts(), pipe->amax_np, sp);
     else
-      ct_scale(st, dp_in, M * L.Cz, sp);
+      spl = ct_scale_lazy(st, dp_in, M * L.Cz, sp);
     if (pipe) pipe->amax_np = 0;
   }
-  transition_bwd(st, B.ptr, M, N, p.p5, nullptr, p.ptr, dp_in, dp_out, sp);
-  triattn_bwd(st, B.tae, true, N, p.p4, pmask, t.pair(b, 3), p.tae, dp_out, dp_out, sp);
-  triattn_bwd(st, B.tas, false, N, p.p3, pmask, t.pair(b, 2), p.tas, dp_out, dp_out, sp);
-  trimul_bwd(st, B.tmi, false, N, p.p2, pmask, t.pair(b, 1), p.tmi, dp_out, dp_out, sp);
+  transition_bwd(st, B.ptr, M, N, p.p5, nullptr, p.ptr, dp_in, dp_out, spl);
+  triattn_bwd(st, B.tae, true, N, p.p4, pmask, t.pair(b, 3), p.tae, dp_out, dp_out, CtScale{sp});
+  triattn_bwd(st, B.tas, false, N, p.p3, pmask, t.pair(b, 2), p.tas, dp_out, dp_out, CtScale{sp});
+  trimul_bwd(st, B.tmi, false, N, p.p2, pmask, t.pair(b, 1), p.tmi, dp_out, dp_out, CtScale{sp});
   trimul_bwd(st, B.tmo, true, N, L.tpl ? f.pin : p.p1, pmask, t.pair(b, 0), p.tmo, dp_out, dp_out,
-             sp);
+             CtScale{sp});
   if (!msa_side) return;
   if (!two) {
     {
       KTimed kt("block.ct_scale", st);
       ct_scale(st, dmsa, (long)S * N * L.Cm, sm);
     }
-    transition_bwd(st, B.mtr, (long)S * N, N, p.m2, nullptr, p.mtr, dmsa, dmsa, sm);
+    transition_bwd(st, B.mtr, (long)S * N, N, p.m2, nullptr, p.mtr, dmsa, dmsa, CtScale{sm});
     msacol_bwd(st, B.col, S, N, p.m1, mmask, nullptr, p.col, dmsa, dmsa, sm);
     // the row attention's pair term is the block's last write of dp_out: its
     // partial maxima serve the next block's pair scale

@@ -18,6 +18,7 @@ namespace bc2n {
 namespace {
 constexpr int CT_SLOTS = 8;
 constexpr int CT_PART = 512;  // partial-maximum blocks (grid of the first pass)
+static_assert(CT_PART <= CT_LAZY, "a lazy scale holds them");
 __device__ __align__(256) float g_ct_slots[CT_SLOTS * 2];
 __device__ __align__(256) float g_ct_part[NUM_LANES * CT_PART];
 __device__ __align__(256) float g_ct_fused[NUM_LANES * CT_FUSED];
@@ -65,8 +66,7 @@ __global__ __launch_bounds__(256) void amax_part_kernel(const float* __restrict_
   if (threadIdx.x == 0) part[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// sc = {s, 1/s}: s = 2^(4 - e) for max|x| in (2^(e-1), 2^e], so s*max|x| is
-// in (8, 16]; s = 1 when x is all zero or its maximum is not finite.
+// sc = {s, 1/s}, s = ct_scale_of(max|x|).
 // One workgroup of 256; four independent loads a thread in flight (up to
 // CT_FUSED partials).
 __global__ __launch_bounds__(256) void amax_final_kernel(const float* __restrict__ part, int np,
@@ -83,12 +83,7 @@ __global__ __launch_bounds__(256) void amax_final_kernel(const float* __restrict
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   if (threadIdx.x == 0) {
-    float s = 1.f;
-    if (m > 0.f && m <= 3.0e38f) {
-      int e = 0;
-      (void)frexpf(m, &e);
-      s = ldexpf(1.f, max(-100, min(100, 4 - e)));
-    }
+    const float s = ct_scale_of(m);
     sc[0] = s;
     sc[1] = 1.f / s;
   }
@@ -99,7 +94,7 @@ float* ct_scale_slot(int k) {
   return ct_ptrs().slots + 2 * k;
 }
 
-void ct_scale(hipStream_t st, const float* x, long n, float* sc) {
+CtScale ct_scale_lazy(hipStream_t st, const float* x, long n, float* sc) {
   if (x == nullptr || n <= 0 || n % 4 != 0 || ((uintptr_t)x & 15))
     throw std::runtime_error("ct_scale: x must be 16-byte aligned with n a positive multiple of 4");
   const CtPtrs p = ct_ptrs();
@@ -107,7 +102,16 @@ void ct_scale(hipStream_t st, const float* x, long n, float* sc) {
   const int blocks = (int)std::min<long>(CT_PART, (n4 + 255) / 256);
   float* part = p.part + (size_t)lane() * CT_PART;
   hipLaunchKernelGGL(amax_part_kernel, dim3(blocks), dim3(256), 0, st, x, n4, part);
-  hipLaunchKernelGGL(amax_final_kernel, dim3(1), dim3(256), 0, st, part, blocks, sc);
+  return {sc, part, blocks};
+}
+
+const float* ct_scale_now(hipStream_t st, const CtScale& c) {
+  if (c.part) hipLaunchKernelGGL(amax_final_kernel, dim3(1), dim3(256), 0, st, c.part, c.np, c.sc);
+  return c.sc;
+}
+
+void ct_scale(hipStream_t st, const float* x, long n, float* sc) {
+  (void)ct_scale_now(st, ct_scale_lazy(st, x, n, sc));
 }
 
 float* ct_fused_parts() { return ct_ptrs().fused + (size_t)lane() * CT_FUSED; }
@@ -116,6 +120,12 @@ void ct_scale_parts(hipStream_t st, const float* part, long np, float* sc) {
   if (!part || !sc || np <= 0 || np > CT_FUSED)
     throw std::runtime_error("ct_scale_parts: 1 to CT_FUSED partial maxima");
   hipLaunchKernelGGL(amax_final_kernel, dim3(1), dim3(256), 0, st, part, (int)np, sc);
+}
+
+CtScale ct_scale_parts_lazy(hipStream_t st, const float* part, long np, float* sc) {
+  if (part && sc && np > 0 && np <= CT_LAZY) return {sc, part, (int)np};
+  ct_scale_parts(st, part, np, sc);
+  return {sc, nullptr, 0};
 }
 
 // ----------------------------------------------------------------- zero fill

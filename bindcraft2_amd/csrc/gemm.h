@@ -959,7 +959,7 @@ struct ALoadRelu16 {
 //   out[src] = dres[src] + rstd * (g - mean(g) - xhat * mean(g * xhat)),
 //   g = gs * gamma * (dy + sum_h dbias[h][m] wb[c][h]),  xhat = (x[src] - mean) * rstd,
 // src = ln_src_row(m, nt) (the transposed orientation when nt > 0), gs =
-// *gmul (the module's inverse cotangent scale; 1 when null).  dres may alias
+// *gmul (the module's inverse cotangent scale; gval when null).  dres may alias
 // out.  16 lanes per row (a DPP row), 8 channels each.  dbias may be given as
 // dbias_nch partials [nch][H][M], added here in chunk order (the attention
 // backward's deferred reduction; the same sums as its reduction kernel).
@@ -972,6 +972,7 @@ struct EpiLnBwd : EpiRows {
   long M;
   int nt;
   int dbias_nch = 1;
+  float gval = 1.f;  // the inverse scale where gmul is null
   // the bias term's per-row head sums, made in the GEMM's prologue
   static constexpr int kProRowFloats = H;
   EpiLnBwd(const float* x_, const float* g_, const float* mu_, const float* rs_, const float* dres_,
@@ -1027,8 +1028,8 @@ struct EpiLnBwd : EpiRows {
     const int lr = tid >> 4, c0 = (tid & 15) * 8;
     float gm[8];
     ld_f8(gamma + c0, gm);
-    if (gmul) {
-      const float gs = *gmul;
+    {
+      const float gs = gmul ? *gmul : gval;
 #pragma unroll
       for (int e = 0; e < 8; ++e) gm[e] *= gs;
     }

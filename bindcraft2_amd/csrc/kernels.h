@@ -145,6 +145,54 @@ void zero_f32(hipStream_t st, float* p, long n);
 // scale; 1, 2: the stack's per-block pair and MSA scales; 3: the template
 // embedding).  No allocation.
 void ct_scale(hipStream_t st, const float* x, long n, float* sc);
+// A scale whose final reduction is left to its first consumer kernel: with
+// part, np partial maxima (CT_LAZY at most) not yet reduced to sc; without, sc
+// holds the scale.  The consumer (CtLoad below) reduces them in every workgroup
+// and writes sc for the kernels after it, so no launch of one workgroup stands
+// between the partials and it (3 to 5 us with the gaps around it).
+struct CtScale {
+  float* sc = nullptr;
+  const float* part = nullptr;
+  int np = 0;
+};
+constexpr int CT_LAZY = 1024;
+CtScale ct_scale_lazy(hipStream_t st, const float* x, long n, float* sc);
+// sc.sc with the scale in it after the launches so far (reduced here if need be).
+const float* ct_scale_now(hipStream_t st, const CtScale& sc);
+// From partials a kernel wrote: lazy up to CT_LAZY, else reduced here.
+CtScale ct_scale_parts_lazy(hipStream_t st, const float* part, long np, float* sc);
+
+// s = 2^(4 - e) for max|x| = m in (2^(e-1), 2^e], so s m is in (8, 16]; 1 when m
+// is 0 or not finite.
+__device__ __forceinline__ float ct_scale_of(float m) {
+  if (!(m > 0.f && m <= 3.0e38f)) return 1.f;
+  int e = 0;
+  (void)frexpf(m, &e);
+  return ldexpf(1.f, max(-100, min(100, 4 - e)));
+}
+// The consumer's side, 256 threads: load() before the kernel's other loads (the
+// memory counter retires in order), scale() where s is needed -- every thread
+// calls it, it holds a barrier -- by one workgroup with `write`.
+struct CtLoad {
+  float m[4];
+  __device__ __forceinline__ void load(const CtScale& c, int tid) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) m[u] = c.part && tid + 256 * u < c.np ? c.part[tid + 256 * u] : 0.f;
+  }
+  __device__ __forceinline__ float scale(const CtScale& c, int tid, bool write) const {
+    if (!c.part) return c.sc[0];
+    __shared__ float red[4];
+    const float w = group_max<64>(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
+    if ((tid & 63) == 0) red[tid >> 6] = w;
+    __syncthreads();
+    const float s = ct_scale_of(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    if (write && tid == 0) {
+      c.sc[0] = s;
+      c.sc[1] = 1.f / s;
+    }
+    return s;
+  }
+};
 float* ct_scale_slot(int k);
 // The same scale from partial maxima a producing kernel wrote (np of them at
 // ct_fused_parts()): the final reduction alone.  ct_fused_parts is the

@@ -70,7 +70,8 @@ struct Args {
   h16* bias;  // [H][M] binary16 in score-fragment order
   const h16* W;
   // SCALED, GATED: dropout table [bn][C] or null, the cotangent scale
-  const float *tbl, *sc;
+  const float* tbl;
+  CtScale sc;
   const h16 *gout, *osave;  // GATED
   h16* dcat;
 };
@@ -218,7 +219,9 @@ kernel(Args a, Epi epi) {
   } else if constexpr (IN == In::SCALED || IN == In::GATED) {
     // two passes' loads in flight at a time (a register budget for four waves)
     constexpr int PF = PASS < 2 ? PASS : 2;
-    const float sm = *a.sc;
+    CtLoad cl;
+    cl.load(a.sc, tid);
+    float sm = 0.f;
     load_b(0);
 #pragma unroll
     for (int p0 = 0; p0 < PASS; p0 += PF) {
@@ -234,6 +237,7 @@ kernel(Args a, Epi epi) {
           os[p] = ld8(a.osave + m * C + c0);
         }
       }
+      if (p0 == 0) sm = cl.scale(a.sc, tid, blockIdx.x == 0);
 #pragma unroll
       for (int p = 0; p < PF; ++p) {
         const int r = (p0 + p) * RPP + fr;
@@ -426,7 +430,7 @@ void launch(hipStream_t st, const Args& a, const Epi& epi) {
   if (a.M <= 0 || a.M % 32 != 0 || a.nout % 32 != 0 || a.nout < 64 || !a.W ||
       ((has_tile<Epi>::value || has_pre<Epi>::value) && a.nout != C) ||
       (H > 0 && (long)a.bn * a.bn != a.M) ||
-      ((IN == In::SCALED || IN == In::GATED) && (a.bn <= 0 || !a.sc)))
+      ((IN == In::SCALED || IN == In::GATED) && (a.bn <= 0 || !a.sc.sc)))
     throw std::runtime_error("row projection: shape");
   auto go = [&](auto rt, auto wc) {
     constexpr int RT = decltype(rt)::value, WC = decltype(wc)::value;

@@ -26,6 +26,11 @@ inline const float* module_scale(hipStream_t st, const float* sc, const float* d
   return s;
 }
 
+// The same with the final reduction left to the module's first kernel.
+inline CtScale module_scale_lazy(hipStream_t st, const CtScale& sc, const float* dout, long n) {
+  return sc.sc ? sc : ct_scale_lazy(st, dout, n, ct_scale_slot(0));
+}
+
 // ---------------------------------------------------------- triangle attention
 // modules.py TriangleAttention (+ Attention with pair bias and gating).
 struct TriAttnW {
@@ -57,7 +62,7 @@ void triattn_fwd_noalloc(hipStream_t st, const TriAttnW& w, bool per_column, int
                          float* pair_out, void* save);
 void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
                  const float* pair_in, const float* mask, const float* tbl,
-                 const void* save, const float* dout, float* din, const float* sc = nullptr);
+                 const void* save, const float* dout, float* din, CtScale sc = {});
 
 // ------------------------------------------------------ triangle multiplication
 // modules.py:1044-1088 (fused projection weights).
@@ -80,7 +85,7 @@ void trimul_fwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
                 const float* mask, const float* tbl, float* pair_out, void* save);
 void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const float* pair_in,
                 const float* mask, const float* tbl, const void* save, const float* dout,
-                float* din, const float* sc = nullptr);
+                float* din, CtScale sc = {});
 
 // ----------------------------------------------------------------- transition
 // modules.py:252-305; pair (rows = N*N) and MSA (rows = S*N) alike.  `nt` is
@@ -99,7 +104,7 @@ void transition_fwd(hipStream_t st, const TransW& w, long rows, int nt, const fl
                     const float* tbl, float* act_out, void* save);
 void transition_bwd(hipStream_t st, const TransW& w, long rows, int nt, const float* act_in,
                     const float* tbl, const void* save, const float* dout, float* din,
-                    const float* sc = nullptr);
+                    CtScale sc = {});
 
 // ------------------------------------------------------------- MSA attention
 struct AttnW {

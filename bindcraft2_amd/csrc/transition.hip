@@ -65,7 +65,7 @@ struct Args {
   int nt;
   const float* x;       // forward: act_in; backward: dout
   const float* tbl;     // dropout table [nt][C] or null
-  const float* sc;      // backward: {s, 1/s}
+  CtScale sc;           // backward: the cotangent scale
   const float *ln_g, *ln_b;
   float *mean, *rstd;   // forward writes, backward reads
   const h16* W1;        // GEMM1's B (n < H, k < C) in fragment order: forward W1^T, backward W2
@@ -124,6 +124,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   {
     const int lr = lane >> 4, c0 = l16 * 8;
     float v[RT][8];
+    CtLoad cl;
+    if constexpr (BWD) cl.load(a.sc, tid);
 #pragma unroll
     for (int p = 0; p < RT; ++p) {
       const long m = min(m0 + p * 16 + w * 4 + lr, M - 1);  // rows past M: in bounds, zeroed below
@@ -156,7 +158,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
     load_b1(0);
     load_b2(0);
+    float sm = 1.f;
     if constexpr (BWD) {
+      sm = cl.scale(a.sc, tid, blockIdx.x == 0);
+      epi.gmul = nullptr;
+      epi.gval = 1.f / sm;  // exact: a power of two
 #pragma unroll
       for (int q = 0; q < NBP; ++q) {
         const int it = tid + 256 * q, r = it / (H / 128), c = it % (H / 128);
@@ -171,7 +177,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       const long m = m0 + r;
       h16x8 o;
       if constexpr (BWD) {
-        const float sm = a.sc[0];
         if constexpr (TBL) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[p][e] *= t[p][e] * sm;
@@ -454,7 +459,7 @@ void transition_fwd(hipStream_t st, const TransW& w, long rows, int nt, const fl
 
 void transition_bwd(hipStream_t st, const TransW& w, long rows, int nt, const float* act_in,
                     const float* tbl, const void* save, const float* dout, float* din,
-                    const float* sc) {
+                    CtScale cs) {
   nonnull(act_in, "transition act"); nonnull(save, "transition save");
   nonnull(dout, "transition dout"); nonnull(din, "transition din");
   const int C = w.C, H = w.C * w.F;
@@ -462,18 +467,18 @@ void transition_bwd(hipStream_t st, const TransW& w, long rows, int nt, const fl
   TransSave<Carver> sv(cv, rows, C, w.F);
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
-  sc = module_scale(st, sc, dout, rows * C);
+  cs = module_scale_lazy(st, cs, dout, rows * C);
   if (C == tf::C && H == tf::H) {
     tf::Args a{};
-    a.M = rows; a.nt = nt; a.x = dout; a.tbl = tbl; a.sc = sc;
+    a.M = rows; a.nt = nt; a.x = dout; a.tbl = tbl; a.sc = cs;
     a.ln_g = w.ln_g; a.mean = sv.mean; a.rstd = sv.rstd;
     a.W1 = w.frag1_b; a.W2 = w.frag2_b; a.bits = sv.hbits;
     tf::fused<true>(st, a,
-                    EpiLnBwd<0>(act_in, w.ln_g, sv.mean, sv.rstd, dout, din, rows, 0, nullptr,
-                                nullptr, sc + 1),
+                    EpiLnBwd<0>(act_in, w.ln_g, sv.mean, sv.rstd, dout, din, rows, 0),
                     "trans.fused_bwd");
     return;
   }
+  const float* sc = ct_scale_now(st, cs);
   Sizer need;
   need.take<h16>((size_t)rows * H);
   need.take<float>((size_t)rows * C);

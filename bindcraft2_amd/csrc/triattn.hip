@@ -424,7 +424,7 @@ void triattn_fwd_noalloc(hipStream_t st, const TriAttnW& w, bool per_column, int
 
 void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
                  const float* pair_in, const float* mask, const float* tbl,
-                 const void* save, const float* dout, float* din, const float* sc) {
+                 const void* save, const float* dout, float* din, CtScale cs) {
   triattn_check(w, N);
   nonnull(pair_in, "triattn pair_in"); nonnull(mask, "triattn mask"); nonnull(save, "triattn save");
   nonnull(dout, "triattn dout"); nonnull(din, "triattn din");
@@ -437,7 +437,9 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   const int nch = attn_bwd_nchunk(N, b.rows_per_chunk);
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
-  sc = module_scale(st, sc, dout, M * C);
+  cs = module_scale_lazy(st, cs, dout, M * C);
+  // the row kernel below reduces a scale still in partials; the GEMM does not
+  const float* sc = w.wo_bfrag ? cs.sc : ct_scale_now(st, cs);
   Sizer need;
   need.take<h16>((size_t)M * HD);           // dO
   need.take<float>((size_t)H * M);           // Dsum
@@ -463,7 +465,7 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   if (w.wo_bfrag) {
     lnproj::Args la{};
     la.M = M; la.nt = per_column ? N : 0; la.bn = N; la.nout = HD;
-    la.x = dout; la.tbl = tbl; la.sc = sc; la.W = w.wo_bfrag;
+    la.x = dout; la.tbl = tbl; la.sc = cs; la.W = w.wo_bfrag;
     KTimed kt(BC2N_TN(C, "triattn.gemm_dout"), st);
     const auto eg = gate(EpiGateBwdT<true>{});
     if (C == 128) lnproj::launch<lnproj::In::SCALED, 128, 0, false>(st, la, eg);

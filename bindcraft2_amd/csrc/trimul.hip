@@ -783,7 +783,7 @@ void trimul_fwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
 
 void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const float* pair_in,
                 const float* mask, const float* tbl, const void* save, const float* dout,
-                float* din, const float* sc) {
+                float* din, CtScale cs) {
   trimul_check(N);
   nonnull(pair_in, "trimul pair_in"); nonnull(mask, "trimul mask"); nonnull(save, "trimul save");
   nonnull(dout, "trimul dout"); nonnull(din, "trimul din");
@@ -793,10 +793,12 @@ void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   TriMulSave<Carver> sv(cv, N, C, I);
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
-  sc = module_scale(st, sc, dout, M * C);
+  cs = module_scale_lazy(st, cs, dout, M * C);
   // I = C = 128 or 64: the tail kernel keeps d(cat)'s [proj|gate] columns on
   // chip; only its gating_linear columns ([M][C]) go through memory
   const bool fused = w.tail_w1 != nullptr;
+  // the row kernel below reduces a scale still in partials; the GEMM does not
+  const float* sc = fused ? cs.sc : ct_scale_now(st, cs);
   const int ldcat = fused ? C : NC, off = fused ? 0 : 4 * I;
   Sizer need;
   need.take<h16>((size_t)M * ldcat);  // dcat
@@ -818,7 +820,7 @@ void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   if (fused) {
     // the centre norm's backward in the epilogue: dT straight from d(tn)
     lnproj::Args la{};
-    la.M = M; la.bn = N; la.nout = I; la.x = dout; la.tbl = tbl; la.sc = sc;
+    la.M = M; la.bn = N; la.nout = I; la.x = dout; la.tbl = tbl; la.sc = cs;
     la.gout = sv.gout; la.osave = sv.osave; la.dcat = dcat; la.W = w.wo_bfrag;
     KTimed kt(BC2N_TN(C, "trimul.gemm_dout_ln"), st);
     auto go = [&](auto ep) {
