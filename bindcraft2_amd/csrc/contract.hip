@@ -71,28 +71,31 @@ __device__ __forceinline__ void store4<h16>(h16* p, f32x4 v) {
 constexpr int SR = 16;  // rows of A per strip
 constexpr int MAXS = 4;  // A strips a workgroup (held in registers)
 
+template <int NB, bool AK, bool BK>
+struct Layout {
+  static constexpr int N = 32 * NB;
+  // LDS: B staging chunk (init only) and the two A strip buffers
+  static constexpr int LDB = BK ? 32 + 8 : N + 8;  // B chunk: [N][32] (K-contig) or [32][N] (k-major)
+  static constexpr int BROWS = BK ? N : 32;
+  static constexpr int LDA = AK ? N + 8 : SR + 8;  // A strip: [16][N] (K-contig) or [N][16] (k-major)
+  static constexpr int AROWS = AK ? SR : N;
+  static constexpr int ABUF = AROWS * LDA;
+  static constexpr int ELEMS = 2 * ABUF + 2 * BROWS * LDB;  // two strips, two staging chunks
+};
+
+// Group grp of channel ch's strips; lds: Layout::ELEMS h16.
 template <int NB, bool AK, bool BK, class OutT>
-__global__ __launch_bounds__(64 * NB) void contract_kernel(const h16* __restrict__ A,
-                                                           const h16* __restrict__ B,
-                                                           OutT* __restrict__ C, long P,
-                                                           int channels, int groups) {
+__device__ __forceinline__ void contract_group(const h16* __restrict__ A, const h16* __restrict__ B,
+                                               OutT* __restrict__ C, long P, int ch, int grp,
+                                               int groups, h16* lds) {
+  using Y = Layout<NB, AK, BK>;
   constexpr int N = 32 * NB;
   constexpr int NT = 64 * NB;      // threads
   constexpr int NS = N / SR;       // strips per channel
-  // LDS: B staging chunk (init only) and the two A strip buffers
-  constexpr int LDB = BK ? 32 + 8 : N + 8;   // B chunk: [N][32] (K-contig) or [32][N] (k-major)
-  constexpr int BROWS = BK ? N : 32;
-  constexpr int LDA = AK ? N + 8 : SR + 8;   // A strip: [16][N] (K-contig) or [N][16] (k-major)
-  constexpr int AROWS = AK ? SR : N;
-  constexpr int ABUF = AROWS * LDA;
-  __shared__ __attribute__((aligned(16))) h16 As[2 * ABUF];
-  __shared__ __attribute__((aligned(16))) h16 Bs[2 * BROWS * LDB];  // two staging chunks
+  constexpr int LDB = Y::LDB, BROWS = Y::BROWS, LDA = Y::LDA, ABUF = Y::ABUF;
+  h16* As = lds;
+  h16* Bs = lds + 2 * ABUF;
   static_assert(SR * N / 8 == NT, "one 16-byte chunk of a strip per thread");
-
-  const long G = (long)channels * groups;
-  const long bid = xcd_block(G);  // (channel, group): a channel's groups share its B plane in L2
-  if (bid >= G) return;
-  const int ch = (int)(bid / groups), grp = (int)(bid % groups);
   const h16* Ap = A + (long)ch * P;
   const h16* Bp = B + (long)ch * P;
   OutT* Cp = C + (long)ch * P;
@@ -199,6 +202,36 @@ __global__ __launch_bounds__(64 * NB) void contract_kernel(const h16* __restrict
   }
 }
 
+template <int NB, bool AK, bool BK, class OutT>
+__global__ __launch_bounds__(64 * NB) void contract_kernel(const h16* A, const h16* B, OutT* C, long P,
+                                                           int channels, int groups) {
+  __shared__ __attribute__((aligned(16))) h16 lds[Layout<NB, AK, BK>::ELEMS];
+  const long G = (long)channels * groups;
+  const long bid = xcd_block(G);  // (channel, group): a channel's groups share its B plane in L2
+  if (bid >= G) return;
+  contract_group<NB, AK, BK, OutT>(A, B, C, P, (int)(bid / groups), (int)(bid % groups), groups, lds);
+}
+
+// Both backward products (dT an operand of both) in one launch: (channel,
+// product, group), so that the two products of a channel share its planes in L2,
+// the gap of some 3 us between them goes, and the groups are sized for both
+// together -- more strips a group, so fewer stagings of B (18.1 us for the two at
+// N = 224, I = 128).  The module's pass, N = 96: 60.7 us in two launches, 57.9 in
+// one; N = 224: 163 and 160.
+template <int NB, bool AK2, bool BK2>
+__global__ __launch_bounds__(64 * NB) void contract_pair_kernel(const h16* A1, const h16* B1, h16* C1,
+                                                                const h16* A2, const h16* B2, h16* C2,
+                                                                long P, int channels, int groups) {
+  constexpr int E1 = Layout<NB, true, false>::ELEMS, E2 = Layout<NB, AK2, BK2>::ELEMS;
+  __shared__ __attribute__((aligned(16))) h16 lds[E1 > E2 ? E1 : E2];
+  const long G = 2L * channels * groups;
+  const long bid = xcd_block(G);
+  if (bid >= G) return;
+  const int grp = (int)(bid % groups), ch = (int)(bid / groups / 2);
+  if (bid / groups % 2 == 0) contract_group<NB, true, false, h16>(A1, B1, C1, P, ch, grp, groups, lds);
+  else contract_group<NB, AK2, BK2, h16>(A2, B2, C2, P, ch, grp, groups, lds);
+}
+
 template <int NB, class OutT>
 void launch(hipStream_t st, bool ak, bool bk, const h16* A, const h16* B, OutT* C, long P,
             int channels, int groups) {
@@ -226,21 +259,47 @@ bool contract_t(hipStream_t st, int N, int channels, const h16* A, bool ak, cons
 
 }  // namespace
 
+// Strip groups a channel: about two workgroups per CU over `planes` products.
+static int strip_groups(int N, int planes) {
+  const int ns = N / SR;
+  return std::max((ns + MAXS - 1) / MAXS,
+                  std::max(1, std::min(ns, (2 * device_cus() + planes - 1) / planes)));
+}
+
 bool trimul_contract(hipStream_t st, int N, int channels, const h16* A, bool a_kcontig,
                      const h16* B, bool b_kcontig, float* Cf, h16* Cb) {
   if (N <= 0 || N % 32 != 0 || N > 256) return false;
   if (((uintptr_t)A & 15) || ((uintptr_t)B & 15) || ((uintptr_t)Cf & 15) || ((uintptr_t)Cb & 7))
     throw std::runtime_error("contract: operands must be 16-byte aligned");
-  int dev = 0, cus = 0;
-  hip_check(hipGetDevice(&dev), "hipGetDevice");
-  hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev),
-            "hipDeviceGetAttribute");
-  // about two workgroups per CU, a channel's strips spread over its groups
-  const int ns = N / SR;
-  const int groups = std::max((ns + MAXS - 1) / MAXS,
-                              std::max(1, std::min(ns, (2 * cus + channels - 1) / channels)));
+  const int groups = strip_groups(N, channels);
   if (Cf) return contract_t<float>(st, N, channels, A, a_kcontig, B, b_kcontig, Cf, groups);
   return contract_t<h16>(st, N, channels, A, a_kcontig, B, b_kcontig, Cb, groups);
+}
+
+bool trimul_contract_pair(hipStream_t st, int N, int channels, const h16* A1, const h16* B1, h16* C1,
+                          const h16* A2, bool a2_kcontig, const h16* B2, bool b2_kcontig, h16* C2) {
+  if (N <= 0 || N % 32 != 0 || N > 256 || (b2_kcontig && !a2_kcontig) || (a2_kcontig && !b2_kcontig))
+    return false;
+  for (const void* p : {(const void*)A1, (const void*)B1, (const void*)C1, (const void*)A2,
+                        (const void*)B2, (const void*)C2})
+    if ((uintptr_t)p & 15) throw std::runtime_error("contract: operands must be 16-byte aligned");
+  const int groups = strip_groups(N, 2 * channels);
+  const dim3 grid(xcd_grid(2L * channels * groups));
+  const long P = (long)N * N;
+  switch (N / 32) {
+#define BC2N_NB(v)                                                                                 \
+  case v:                                                                                          \
+    if (b2_kcontig)                                                                                \
+      hipLaunchKernelGGL((contract_pair_kernel<v, true, true>), grid, dim3(64 * v), 0, st, A1, B1, \
+                         C1, A2, B2, C2, P, channels, groups);                                     \
+    else                                                                                           \
+      hipLaunchKernelGGL((contract_pair_kernel<v, false, false>), grid, dim3(64 * v), 0, st, A1,   \
+                         B1, C1, A2, B2, C2, P, channels, groups);                                 \
+    return true;
+    BC2N_NB(1) BC2N_NB(2) BC2N_NB(3) BC2N_NB(4) BC2N_NB(5) BC2N_NB(6) BC2N_NB(7) BC2N_NB(8)
+#undef BC2N_NB
+    default: return false;
+  }
 }
 
 }  // namespace bc2n

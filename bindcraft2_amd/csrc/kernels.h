@@ -131,6 +131,12 @@ void ln_f32_rows_bwd(hipStream_t st, const float* dy, const float* x, long M, in
 bool trimul_contract(hipStream_t st, int N, int channels, const h16* A, bool a_kcontig,
                      const h16* B, bool b_kcontig, float* Cf, h16* Cb);
 
+// The two backward products in one launch: C1 = A1 B1 with A1 K-contiguous and
+// B1 k-major, and C2 = A2 B2 with both operands k-major or both K-contiguous.
+// False (nothing launched) outside the same range.
+bool trimul_contract_pair(hipStream_t st, int N, int channels, const h16* A1, const h16* B1, h16* C1,
+                          const h16* A2, bool a2_kcontig, const h16* B2, bool b2_kcontig, h16* C2);
+
 // p[0..n) = 0 by a kernel (graph-capture safe, unlike hipMemsetAsync).
 void zero_f32(hipStream_t st, float* p, long n);
 

@@ -858,8 +858,15 @@ void trimul_bwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
       b.A = sv.left; b.a_sm = N; b.a_sk = 1;
       b.B = dT; b.b_sn = N; b.b_sk = 1;
     }
-    contract<h16>(st, a, dL, BC2N_TN(C, "trimul.contract_bwd"));
-    contract<h16>(st, b, dR, BC2N_TN(C, "trimul.contract_bwd"));
+    bool one = false;
+    if (N <= 256) {
+      KTimed kt(BC2N_TN(C, "trimul.contract_bwd"), st);
+      one = trimul_contract_pair(st, N, I, a.A, a.B, dL, b.A, b.a_sk == 1, b.B, b.b_sk == 1, dR);
+    }
+    if (!one) {
+      contract<h16>(st, a, dL, BC2N_TN(C, "trimul.contract_bwd"));
+      contract<h16>(st, b, dR, BC2N_TN(C, "trimul.contract_bwd"));
+    }
   }
   if (fused) {
     TailArgs t;
