@@ -954,19 +954,19 @@ struct ALoadRelu16 {
 
 
 // LayerNorm backward fused into the GEMM that produces its cotangent dy (the
-// d(LN output) of a module's input projections), C = BN = 128 channels, with
+// d(LN output) of a module's input projections), C = BN = 128 or 64 channels, with
 // the residual cotangent added:
 //   out[src] = dres[src] + rstd * (g - mean(g) - xhat * mean(g * xhat)),
 //   g = gs * gamma * (dy + sum_h dbias[h][m] wb[c][h]),  xhat = (x[src] - mean) * rstd,
 // src = ln_src_row(m, nt) (the transposed orientation when nt > 0), gs =
 // *gmul (the module's inverse cotangent scale; gval when null).  dres may alias
-// out.  16 lanes per row (a DPP row), 8 channels each.  dbias may be given as
+// out.  C / 8 lanes per row (within a DPP row), 8 channels each.  dbias may be given as
 // dbias_nch partials [nch][H][M], added here in chunk order (the attention
 // backward's deferred reduction; the same sums as its reduction kernel).
-template <int H>
+template <int H, int C_ = 128>
 struct EpiLnBwd : EpiRows {
   static constexpr bool kRowBlock = true;
-  static constexpr int C = 128;
+  static constexpr int C = C_, LPR = C / 8, RPP = 256 / LPR;  // lanes a row, rows a pass
   const float *x, *gamma, *mean, *rstd, *dres, *dbias, *wb, *gmul;
   float* out;
   long M;
@@ -1025,7 +1025,7 @@ struct EpiLnBwd : EpiRows {
   template <int WM>
   __device__ __forceinline__ void block(int, long mb, const float* T, int ldt, int tid,
                                         const float* pro = nullptr) const {
-    const int lr = tid >> 4, c0 = (tid & 15) * 8;
+    const int lr = tid / LPR, c0 = tid % LPR * 8;
     float gm[8];
     ld_f8(gamma + c0, gm);
     {
@@ -1048,16 +1048,16 @@ struct EpiLnBwd : EpiRows {
     // before its arithmetic: one memory round trip a group, not one a row
     // (the GEMM's 64-row halves take 4 rows a lane group; the transition's
     // 48-row tile keeps one, its register budget allows no more)
-    constexpr int G = WM % 64 == 0 ? 4 : 1;
-    static_assert(WM % (16 * G) == 0, "rows a pass");
+    constexpr int G = WM % (4 * RPP) == 0 ? 4 : WM % (2 * RPP) == 0 ? 2 : 1;
+    static_assert(WM % (RPP * G) == 0, "rows a pass");
 #pragma unroll 1
-    for (int r0 = 0; r0 < WM; r0 += 16 * G) {
+    for (int r0 = 0; r0 < WM; r0 += RPP * G) {
       float xv[G][8], dr[G][8], db[G][H > 0 ? H : 1], mu[G], rs[G];
       long src[G];
 #pragma unroll
       for (int q = 0; q < G; ++q) {
         // rows past M read row M - 1 (in bounds) and store nothing
-        const long m = min(mb + r0 + 16 * q + lr, M - 1);
+        const long m = min(mb + r0 + RPP * q + lr, M - 1);
         src[q] = ln_src_row(m, nt);
         ld_f8(x + src[q] * C + c0, xv[q]);
         ld_f8(dres + src[q] * C + c0, dr[q]);
@@ -1065,7 +1065,7 @@ struct EpiLnBwd : EpiRows {
 #pragma unroll
           for (int h = 0; h < H; ++h) {
             if (pro) {
-              db[q][h] = pro[(r0 + 16 * q + lr) * H + h];
+              db[q][h] = pro[(r0 + RPP * q + lr) * H + h];
             } else if (dbias_nch == 1) {
               db[q][h] = dbias[(long)h * M + m];
             } else {
@@ -1080,9 +1080,9 @@ struct EpiLnBwd : EpiRows {
       }
 #pragma unroll
       for (int q = 0; q < G; ++q) {
-        if (mb + r0 + 16 * q + lr >= M) continue;  // the row's 16 lanes leave together
+        if (mb + r0 + RPP * q + lr >= M) continue;  // the row's lanes leave together
         float g[8];
-        ld_f8(T + (r0 + 16 * q + lr) * ldt + c0, g);
+        ld_f8(T + (r0 + RPP * q + lr) * ldt + c0, g);
         if constexpr (H > 0) {
 #pragma unroll
           for (int h = 0; h < H; ++h)
@@ -1097,8 +1097,8 @@ struct EpiLnBwd : EpiRows {
           sg += g[e];
           sgx += g[e] * xv[q][e];
         }
-        sg = group_sum<16>(sg) * (1.f / C);
-        sgx = group_sum<16>(sgx) * (1.f / C);
+        sg = group_sum<LPR>(sg) * (1.f / C);
+        sgx = group_sum<LPR>(sgx) * (1.f / C);
 #pragma unroll
         for (int e = 0; e < 8; ++e) dr[q][e] += rs[q] * (g[e] - sg - xv[q][e] * sgx);
         st_f8(out + src[q] * C + c0, dr[q]);

@@ -4,9 +4,9 @@
 //      -> GEMM (F*C -> C) + bias, fused residual (+ shared dropout table)
 // Backward: dh = ((tbl*dout) . W2^T) * (h > 0), the dropout scale applied as
 // the GEMM loads A; dxn = dh . W1^T; LN backward accumulated into din.
-// The pair transition (C = 128, F = 4) runs each direction as one kernel
-// (tf::fused_kernel, the hidden never leaves the CU); the MSA and template
-// widths as LN + two GEMMs.
+// The pair transition (C = 128, F = 4) and the template stack's (C = 64, F = 2)
+// run each direction as one kernel (tf::fused_kernel, the hidden never leaves the
+// CU); the MSA's width as LN + two GEMMs.
 //
 // The backward's ReLU mask is h > 0, and every pre-activation that rounding
 // moves across zero flips a mask entry against the exact model: with bf16
@@ -32,14 +32,15 @@ struct TransSave {
 };
 
 // ------------------------------------------------------------ fused MLP
-// The pair transition (C = 128, hidden H = 512) as one kernel a direction.
+// The pair transition (C = 128, hidden H = 512) and the template stack's (64,
+// 128) as one kernel a direction.
 // A workgroup owns BM = 16 RT rows.  Its input tile -- the LayerNorm output
 // forward, the scaled cotangent backward -- stays in LDS as binary16, and the
 // hidden layer is made and consumed 128 columns at a time: GEMM1 of the
 // chunk, bias + ReLU (forward) or the kept mask (backward), the binary16
 // chunk written k-major to LDS, GEMM2 accumulating into the workgroup's
-// BM x 128 output.  The hidden never leaves the CU.  The 4 waves split the
-// 128 columns of both products (32 each) over all BM rows, so every weight
+// BM x C output.  The hidden never leaves the CU.  The 4 waves split the
+// columns of both products over all BM rows, so every weight
 // fragment is read from L2 once per workgroup, prefetched one chunk ahead.
 //   forward:  xn = LN(x); h = relu(xn . W1 + b1); out = x + tbl * (h . W2 + b2)
 //   backward: g = h16(s * tbl * dout); dh = (g . W2^T) * [h > 0];
@@ -47,9 +48,11 @@ struct TransSave {
 // Both products take binary16 operands with f32 accumulation, rounded where
 // the unfused GEMMs round (the same elementwise formulas).
 namespace tf {
-constexpr int C = 128, H = 512, HC = 128, NCH = H / HC;
+constexpr int HC = 128;  // hidden columns a chunk
+// The widths fused: the pair track's (C = 128, F = 4) and the template stack's.
+constexpr bool width(int C, int H) { return (C == 128 && H == 512) || (C == 64 && H == 128); }
 
-template <int RT>
+template <int C, int H, int RT>
 struct Geom {
   static constexpr int BM = 16 * RT;
   static constexpr int LDX = C + 8;  // xs[BM][LDX]: a 16-row 16-byte read covers every bank once
@@ -75,9 +78,13 @@ struct Args {
 };
 
 // TBL (backward only): the cotangent is scaled by the dropout table a.tbl.
-template <int RT, bool BWD, bool TBL, class Epi>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void fused_kernel(Args a, Epi epi) {
-  using G = Geom<RT>;
+template <int C, int H, int RT, bool BWD, bool TBL, class Epi>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(C == 128 ? 3 : 4, C == 128 ? 3 : 8))) void
+fused_kernel(Args a, Epi epi) {
+  using G = Geom<C, H, RT>;
+  constexpr int NCH = H / HC, KS = C / 32, JJ = C / 64;  // chunks; GEMM1's K steps; output tiles a wave
+  constexpr int LPR = C / 8, RPP = 256 / LPR, PASS = G::BM / RPP;  // front: lanes a row, rows a pass
+  static_assert(G::BM % RPP == 0, "whole passes");
   constexpr int BM = G::BM, LDX = G::LDX, LDH = G::LDH, LDT = G::LDT;
   __shared__ __align__(16) char smem[G::BYTES];
   h16* xs = reinterpret_cast<h16*>(smem);
@@ -88,23 +95,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, l16 = lane & 15;
   const long M = a.M, m0 = (long)blockIdx.x * BM;
 
-  h16x8 b1[4][2];
-  h16x8 b2[4][2];
+  h16x8 b1[KS][2];
+  h16x8 b2[4][JJ];
   float bb[2] = {0.f, 0.f};  // forward: b1 of this lane's two hidden columns
   // Workgroups walk the hidden chunks from different starting chunks, so the
   // many workgroups in flight do not all read the same weight lines at once.
   const int rot = blockIdx.x & (NCH - 1);
-  // fragment f = ((j * 4 + w) * 2 + jj) * 4 + ks of a product's B operand is
-  // 64 lanes x 8 binary16, contiguous: one 1 KB wave load
-  auto frag = [&](const h16* F, int j, int jj, int ks) {
-    return ld8(F + ((long)(((j * 4 + w) * 2 + jj) * 4 + ks) * 64 + lane) * 8);
-  };
+  // a fragment of a product's B operand is 64 lanes x 8 binary16, contiguous:
+  // one 1 KB wave load
+  auto frag = [&](const h16* F, int f) { return ld8(F + ((long)f * 64 + lane) * 8); };
   auto load_b1 = [&](int jl) {
     const int j = (jl + rot) & (NCH - 1);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) b1[ks][jj] = frag(a.W1, j, jj, ks);
+      for (int jj = 0; jj < 2; ++jj) b1[ks][jj] = frag(a.W1, ((j * 4 + w) * 2 + jj) * KS + ks);
     if constexpr (!BWD) {
       bb[0] = a.b1[j * HC + 32 * w + l16];
       bb[1] = a.b1[j * HC + 32 * w + 16 + l16];
@@ -115,28 +120,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) b2[ks][jj] = frag(a.W2, j, jj, ks);
+      for (int jj = 0; jj < JJ; ++jj) b2[ks][jj] = frag(a.W2, ((j * 4 + w) * JJ + jj) * 4 + ks);
   };
 
-  // front: the binary16 input tile, 16 lanes a row, 8 channels a lane.  Its
+  // front: the binary16 input tile, 8 channels a lane.  Its
   // loads go out first, so that waiting for them does not wait for the
   // weight fragments behind them (the memory counter retires in order).
   {
-    const int lr = lane >> 4, c0 = l16 * 8;
-    float v[RT][8];
+    const int lr = tid / LPR, lp = tid % LPR, c0 = lp * 8;
+    float v[PASS][8];
     CtLoad cl;
     if constexpr (BWD) cl.load(a.sc, tid);
 #pragma unroll
-    for (int p = 0; p < RT; ++p) {
-      const long m = min(m0 + p * 16 + w * 4 + lr, M - 1);  // rows past M: in bounds, zeroed below
+    for (int p = 0; p < PASS; ++p) {
+      const long m = min(m0 + p * RPP + lr, M - 1);  // rows past M: in bounds, zeroed below
       ld_f8(a.x + m * C + c0, v[p]);
     }
     float gm[8], bt[8];
-    float t[TBL ? RT : 1][8];
+    float t[TBL ? PASS : 1][8];
     if constexpr (TBL) {
 #pragma unroll
-      for (int p = 0; p < RT; ++p) {
-        const long m = min(m0 + p * 16 + w * 4 + lr, M - 1);
+      for (int p = 0; p < PASS; ++p) {
+        const long m = min(m0 + p * RPP + lr, M - 1);
         ld_f8(a.tbl + (m % a.nt) * C + c0, t[p]);
       }
     }
@@ -172,8 +177,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       }
     }
 #pragma unroll
-    for (int p = 0; p < RT; ++p) {
-      const int r = p * 16 + w * 4 + lr;
+    for (int p = 0; p < PASS; ++p) {
+      const int r = p * RPP + lr;
       const long m = m0 + r;
       h16x8 o;
       if constexpr (BWD) {
@@ -190,17 +195,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         float s = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) s += v[p][e];
-        const float mu = group_sum<16>(s) / C;
+        const float mu = group_sum<LPR>(s) / C;
         float d2 = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float d = v[p][e] - mu;
           d2 += d * d;
         }
-        const float rs = rsqrtf(group_sum<16>(d2) / C + LN_EPS);
+        const float rs = rsqrtf(group_sum<LPR>(d2) / C + LN_EPS);
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = (h16)((v[p][e] - mu) * rs * gm[e] + bt[e]);
-        if (l16 == 0 && m < M) {
+        if (lp == 0 && m < M) {
           a.mean[m] = mu;
           a.rstd[m] = rs;
         }
@@ -211,11 +216,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   }
   __syncthreads();
 
-  f32x4 ao[RT][2];
+  f32x4 ao[RT][JJ];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) ao[i][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < JJ; ++jj) ao[i][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
@@ -227,7 +232,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) ah[i][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+    for (int ks = 0; ks < KS; ++ks) {
       h16x8 af[RT];
 #pragma unroll
       for (int i = 0; i < RT; ++i) af[i] = ld8(xs + (i * 16 + l16) * LDX + ks * 32 + 8 * g);
@@ -285,14 +290,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       }
     }
     __syncthreads();
-    // GEMM2: output columns 32w + 16jj + l16, K = this chunk's hidden columns
+    // GEMM2: output columns 16 (JJ w + jj) + l16, K = this chunk's hidden columns
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       h16x8 af[RT];
 #pragma unroll
       for (int i = 0; i < RT; ++i) af[i] = gemm_tr8(hs, LDH, ks * 32, i * 16, lane);
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
+      for (int jj = 0; jj < JJ; ++jj)
 #pragma unroll
         for (int i = 0; i < RT; ++i) ao[i][jj] = mfma16x16x32(af[i], b2[ks][jj], ao[i][jj]);
     }
@@ -303,10 +308,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
+    for (int jj = 0; jj < JJ; ++jj)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        T[(i * 16 + 4 * g + r) * LDT + 32 * w + 16 * jj + l16] = ao[i][jj][r];
+        T[(i * 16 + 4 * g + r) * LDT + 16 * (JJ * w + jj) + l16] = ao[i][jj][r];
   if constexpr (!BWD) {
     for (int it = tid; it < BM * (H / 128); it += 256) {
       const int r = it / (H / 128), q = it % (H / 128);
@@ -331,46 +336,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   }
 }
 
-constexpr int kRT = 3;  // 48-row tiles (64 and 32 measured slower)
-
-// B operands in the kernel's fragment order.  Lane l = 16 g + c of fragment
-// (j, w, jj, ks) holds B[n][k0 + s(e)], e = 0..7, n = column j*HC + 32w +
-// 16jj + c of the product; GEMM1 (A K-contiguous in LDS) takes the K-slots
-// k0 = ks*32, s(e) = 8g + e; GEMM2 (A read transposed) takes k0 = j*HC +
-// ks*32, s(e) = 4g + e (e < 4) and 16 + 4g + e - 4.  GEMM2's columns are the
-// C outputs, so its n drops the j*HC term and its k carries it.
+// B operands in the kernel's fragment order.  Lane l = 16 g + c of fragment f
+// holds B[n][k0 + s(e)], e = 0..7.  GEMM1, f = ((j*4 + w)*2 + jj)*(C/32) + ks
+// (A K-contiguous in LDS): n = j*HC + 32w + 16jj + c, k0 = ks*32, s(e) = 8g + e;
+// GEMM2, f = ((j*4 + w)*(C/64) + jj)*4 + ks (A read transposed): n = 16 (C/64 w +
+// jj) + c, k0 = j*HC + ks*32, s(e) = 4g + e (e < 4) and 16 + 4g + e - 4.
 template <class B>
-std::vector<h16> make_frags(bool second, B b) {
+std::vector<h16> make_frags(bool second, int C, int H, B b) {
   std::vector<h16> f((size_t)H * C);
-  for (int j = 0; j < NCH; ++j)
+  const int nj = second ? C / 64 : 2, nks = second ? 4 : C / 32;
+  size_t o = 0;
+  for (int j = 0; j < H / HC; ++j)
     for (int w = 0; w < 4; ++w)
-      for (int jj = 0; jj < 2; ++jj)
-        for (int ks = 0; ks < 4; ++ks)
+      for (int jj = 0; jj < nj; ++jj)
+        for (int ks = 0; ks < nks; ++ks)
           for (int l = 0; l < 64; ++l)
             for (int e = 0; e < 8; ++e) {
               const int g = l >> 4, c = l & 15;
-              const int n = (second ? 0 : j * HC) + 32 * w + 16 * jj + c;
+              const int n = second ? 16 * (nj * w + jj) + c : j * HC + 32 * w + 16 * jj + c;
               const int k = second ? j * HC + ks * 32 + (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4)
                                    : ks * 32 + 8 * g + e;
-              f[((size_t)(((j * 4 + w) * 2 + jj) * 4 + ks) * 64 + l) * 8 + e] = (h16)b(n, k);
+              f[o++] = (h16)b(n, k);
             }
   return f;
 }
 
-template <bool BWD, class Epi>
+template <int C, int RT, bool BWD, class Epi>
 void fused(hipStream_t st, const Args& a, const Epi& epi, const char* name) {
   if (a.M <= 0 || a.M > (1L << 30)) throw std::runtime_error("transition: rows out of range");
   if (a.tbl && a.nt <= 0) throw std::runtime_error("transition: dropout table needs nt > 0");
+  constexpr int H = C == 128 ? 512 : 128;
   KTimed kt(name, st);
-  const long nb = (a.M + Geom<kRT>::BM - 1) / Geom<kRT>::BM;
+  const long nb = (a.M + Geom<C, H, RT>::BM - 1) / Geom<C, H, RT>::BM;
   bool tbl = false;
   if constexpr (BWD) tbl = a.tbl != nullptr;
   if (tbl)
-    hipLaunchKernelGGL((fused_kernel<kRT, BWD, BWD, Epi>), dim3((unsigned)nb), dim3(256), 0, st, a,
-                       epi);
-  else
-    hipLaunchKernelGGL((fused_kernel<kRT, BWD, false, Epi>), dim3((unsigned)nb), dim3(256), 0, st,
+    hipLaunchKernelGGL((fused_kernel<C, H, RT, BWD, BWD, Epi>), dim3((unsigned)nb), dim3(256), 0, st,
                        a, epi);
+  else
+    hipLaunchKernelGGL((fused_kernel<C, H, RT, BWD, false, Epi>), dim3((unsigned)nb), dim3(256), 0,
+                       st, a, epi);
+}
+
+// Rows a workgroup.  C = 128: 48 (64 and 32 measured slower).  C = 64: 32 up to
+// 128 rows a CU, so that every CU has workgroups to overlap, then 64, which read
+// each weight fragment half as often (forward / backward: N = 64 2.0 / 2.4 us
+// with 32, 3.2 / 3.5 with 64; N = 128 2.7 / 4.8 and 3.7 / 5.2; N = 192 5.9 / 9.8
+// and 6.5 / 9.5; N = 256 9.0 / 11.3 and 8.6 / 9.6).  As LayerNorm and two
+// products a direction, N = 192 took 20.9 / 23.2 in three launches each.
+template <int C, bool BWD, class Epi>
+void fused(hipStream_t st, const Args& a, const Epi& epi, const char* name) {
+  if constexpr (C == 128) fused<C, 3, BWD>(st, a, epi, name);
+  else if (a.M <= 128L * device_cus()) fused<C, 2, BWD>(st, a, epi, name);
+  else fused<C, 4, BWD>(st, a, epi, name);
 }
 }  // namespace tf
 
@@ -391,20 +409,20 @@ TransW transition_weights(WeightStore& ws, const std::string& P) {
   w.w1_t = ws.derived<h16>("trans.w1_t:" + P, [&] { return transpose_h16(w1.data.data(), C, H); });
   w.w2 = ws.derived<h16>("trans.w2:" + P, [&] { return to_h16(w2.data); });
   w.w2_t = ws.derived<h16>("trans.w2_t:" + P, [&] { return transpose_h16(w2.data.data(), H, C); });
-  if (C == tf::C && H == tf::H) {
+  if (tf::width(C, H)) {
     const float* a1 = w1.data.data();  // [C][H]
     const float* a2 = w2.data.data();  // [H][C]
     w.frag1_f = ws.derived<h16>("trans.frag1_f:" + P, [&] {
-      return tf::make_frags(false, [&](int n, int k) { return a1[(size_t)k * H + n]; });
+      return tf::make_frags(false, C, H, [&](int n, int k) { return a1[(size_t)k * H + n]; });
     });
     w.frag2_f = ws.derived<h16>("trans.frag2_f:" + P, [&] {
-      return tf::make_frags(true, [&](int n, int k) { return a2[(size_t)k * C + n]; });
+      return tf::make_frags(true, C, H, [&](int n, int k) { return a2[(size_t)k * C + n]; });
     });
     w.frag1_b = ws.derived<h16>("trans.frag1_b:" + P, [&] {
-      return tf::make_frags(false, [&](int n, int k) { return a2[(size_t)n * C + k]; });
+      return tf::make_frags(false, C, H, [&](int n, int k) { return a2[(size_t)n * C + k]; });
     });
     w.frag2_b = ws.derived<h16>("trans.frag2_b:" + P, [&] {
-      return tf::make_frags(true, [&](int n, int k) { return a1[(size_t)n * H + k]; });
+      return tf::make_frags(true, C, H, [&](int n, int k) { return a1[(size_t)n * H + k]; });
     });
   }
   return w;
@@ -423,13 +441,14 @@ void transition_fwd(hipStream_t st, const TransW& w, long rows, int nt, const fl
   const int C = w.C, H = w.C * w.F;
   Carver cv(save);
   TransSave<Carver> sv(cv, rows, C, w.F);
-  if (C == tf::C && H == tf::H) {
+  if (tf::width(C, H)) {
     tf::Args a{};
     a.M = rows; a.nt = nt; a.x = act_in; a.tbl = tbl;
     a.ln_g = w.ln_g; a.ln_b = w.ln_b; a.mean = sv.mean; a.rstd = sv.rstd;
     a.W1 = w.frag1_f; a.W2 = w.frag2_f; a.b1 = w.b1; a.bits = sv.hbits;
-    tf::fused<false>(st, a, EpiResidualRows(act_in, act_out, w.b2, tbl, nt, C, false),
-                     "trans.fused_fwd");
+    const EpiResidualRows res(act_in, act_out, w.b2, tbl, nt, C, false);
+    if (C == 128) tf::fused<128, false>(st, a, res, BC2N_TN(C, "trans.fused_fwd"));
+    else tf::fused<64, false>(st, a, res, BC2N_TN(C, "trans.fused_fwd"));
     return;
   }
   Arena& ar = arena();
@@ -468,14 +487,19 @@ void transition_bwd(hipStream_t st, const TransW& w, long rows, int nt, const fl
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
   cs = module_scale_lazy(st, cs, dout, rows * C);
-  if (C == tf::C && H == tf::H) {
+  if (tf::width(C, H)) {
     tf::Args a{};
     a.M = rows; a.nt = nt; a.x = dout; a.tbl = tbl; a.sc = cs;
     a.ln_g = w.ln_g; a.mean = sv.mean; a.rstd = sv.rstd;
     a.W1 = w.frag1_b; a.W2 = w.frag2_b; a.bits = sv.hbits;
-    tf::fused<true>(st, a,
-                    EpiLnBwd<0>(act_in, w.ln_g, sv.mean, sv.rstd, dout, din, rows, 0),
-                    "trans.fused_bwd");
+    auto go = [&](auto c) {
+      constexpr int CC = decltype(c)::value;
+      tf::fused<CC, true>(st, a,
+                          EpiLnBwd<0, CC>(act_in, w.ln_g, sv.mean, sv.rstd, dout, din, rows, 0),
+                          BC2N_TN(C, "trans.fused_bwd"));
+    };
+    if (C == 128) go(std::integral_constant<int, 128>());
+    else go(std::integral_constant<int, 64>());
     return;
   }
   const float* sc = ct_scale_now(st, cs);
