@@ -36,6 +36,7 @@ each kind, the trunk step.
 import argparse
 import json
 import os
+import re
 import sys
 import tempfile
 import time
@@ -95,12 +96,14 @@ def kernel_model(name, n):
         "attn_bwd_dkv": (8 * n ** 3 * c, m * (8 * c + 4 * c + 4 * h + 8 * h + 4 + 4 * h)),
         # left, right read (binary16); T written (f32)
         "trimul.contract_fwd": (2 * c * n ** 3, m * (4 * c + 4 * c)),
-        # dT and one operand read, dL or dR written (binary16)
-        "trimul.contract_bwd": (2 * c * n ** 3, m * 6 * c),
+        # up to N = 256 both products a launch: dT, left and right read, dL and dR
+        # written (binary16); beyond, dT and one operand read, dL or dR written
+        "trimul.contract_bwd": (4 * c * n ** 3, m * 10 * c) if n <= 256 else
+                               (2 * c * n ** 3, m * 6 * c),
         "triattn.gemm_qkvg": (gemm(c, 4 * c), m * (2 * c + 8 * c)),
-        # input LayerNorm + bias heads + q|k|v|g projection in one kernel (C = 128):
+        # input LayerNorm + bias heads + q|k|v|g projection in one kernel:
         # pair read, xn + statistics + bias + qkvg written
-        # input LayerNorm + the 4I + C projection columns in one kernel (C = 128)
+        # input LayerNorm + the 4I + C projection columns in one kernel
         "trimul.ln_proj": (gemm(c, 5 * c), m * (4 * c + 2 * c + 8 + 4 + 2 * 2 * c + 2 * c)),
         "triattn.ln_qkvg": (gemm(c, 4 * c), m * (4 * c + 2 * c + 8 + 4 * h + 8 * c)),
         "triattn.gemm_out": (gemm(c, c), m * (2 * c + 4 * c + 4 * c)),
@@ -109,7 +112,7 @@ def kernel_model(name, n):
         "trimul.gemm_proj": (gemm(c, 5 * c), m * (2 * c + 4 * c + 2 * c + 4)),
         "trimul.proj_bwd": (gemm(c, 4 * c), m * (2 * c + 4 * c + 4 + 8 * c)),
         "trimul.gemm_out": (gemm(c, c), m * (2 * c + 2 * c + 4 * c + 2 * c + 4 * c)),
-        # centre norm + output projection in one kernel (C = 128): T read (f32),
+        # centre norm + output projection in one kernel: T read (f32),
         # statistics, then the output epilogue's traffic
         "trimul.ln_out": (gemm(c, c), m * (4 * c + 8 + 2 * c + 4 * c + 2 * c + 4 * c)),
         "trimul.gemm_dout": (gemm(c, c), m * (4 * c + 2 * c + 2 * c + 4 * c + 2 * c)),
@@ -124,7 +127,7 @@ def kernel_model(name, n):
         "trimul.gemm_dx_ln": (gemm(5 * c, c), m * (10 * c + 12 * c + 8)),
         "triattn.gemm_dx_ln": (gemm(4 * c, c), m * (8 * c + 12 * c + 4 * h + 8)),
         "trans.gemm_dx_ln": (gemm(f * c, c), m * (2 * f * c + 12 * c + 8)),
-        # the pair transition as one kernel a direction (C = 128): x read, out
+        # the pair and template transitions as one kernel a direction: x read, out
         # written, LN statistics, the hidden's mask bits; the hidden stays on chip
         "trans.fused_fwd": (gemm(c, f * c) + gemm(f * c, c), m * (4 * c + 4 * c + 8 + f * c // 8)),
         "trans.fused_bwd": (gemm(c, f * c) + gemm(f * c, c),
@@ -298,12 +301,12 @@ def traffic_of(kernel, n):
     # the triangle-attention launches are the head-width-32 instantiation (the
     # row-chunk forms for N <= 256); other timer names map to no one symbol
     nb = n // 32
-    syms = {"attn_fwd": [f"attn_fwd_rows<32, {nb}>", f"attn_fwd<32, {nb}, 8>"],
-            "attn_bwd_dq": [f"attn_bwd_dq_rows<32, {nb}>", f"attn_bwd_dq<32, {nb}, 8>"],
+    syms = {"attn_fwd": [f"attn_fwd_rows<32, {nb}>", *(f"attn_fwd<32, {nb}, {cb}>" for cb in (2, 3))],
+            "attn_bwd_dq": [f"attn_bwd_dq_rows<32, {nb}>", f"attn_bwd_dq<32, {nb}, 2>"],
             "attn_bwd_dkv": [f"attn_bwd_dkv_lds<{nb}>", f"attn_bwd_dkv_lds8<{nb}>",
                              f"attn_bwd_dkv<32, {nb}, {8 if nb > 8 else 4}, "
                              f"{8 if nb > 24 else 4 if nb > 8 else 2}>"],
-            "trimul.tail_bwd": ["trimul_tail", "_ZN4bc2n12_GLOBAL__N_118trimul_tail_kernelENS0_8TailArgsE"]}.get(kernel, [kernel])
+            "trimul.tail_bwd": ["trimul_tail<128, 3>"]}.get(kernel, [kernel])
     for sym in syms:
         k = summ["kernels"].get(sym)
         if k is not None:
@@ -312,18 +315,17 @@ def traffic_of(kernel, n):
     # mangled); the contraction's output type tells forward from backward
     pat = {"trimul.proj_bwd": r"EpiTrimulProjBwd",
            "trimul.gemm_proj": r"gemm.*EpiTrimulProj(?!Bwd)",
-           "trimul.ln_proj": r"^kernel<0, true, EpiTrimulProj\b|lnproj.*EpiTrimulProj",
-           "triattn.ln_qkvg": r"^kernel<4, false, EpiScaledCols\b|lnproj.*EpiScaledCols",
-           "trans.fused_fwd": r"^fused<.*EpiResidualRows|fused_kernel.*EpiResidualRows",
-           "trans.fused_bwd": r"^fused<.*EpiLnBwd|fused_kernel.*EpiLnBwd",
+           "trimul.ln_proj": r"^kernel<.*128, .*EpiTrimulProj\b|lnproj.*EpiTrimulProj",
+           "triattn.ln_qkvg": r"^kernel<.*128, .*EpiScaledCols\b|lnproj.*EpiScaledCols",
+           "trans.fused_fwd": r"^fused<128, .*EpiResidualRows|fused_kernel.*EpiResidualRows",
+           "trans.fused_bwd": r"^fused<128, .*EpiLnBwd|fused_kernel.*EpiLnBwd",
            "trimul.gemm_out": r"EpiTrimulOut",
            "trimul.ln_out": r"EpiTrimulOut",
-           "triattn.gemm_dx_ln": r"EpiLnBwd<4>|EpiLnBwdILi4E",
+           "triattn.gemm_dx_ln": r"EpiLnBwd<4, 128>|EpiLnBwdILi4E|triattn_dx",
            "trimul.contract_fwd": rf"contract(_kernel)?(<{nb}, .*float>|ILi{nb}E.*fEE)",
-           "trimul.contract_bwd": rf"contract(_kernel)?(<{nb}, .*_Float16>|ILi{nb}E.*DF16_EE)"}.get(kernel)
+           "trimul.contract_bwd": rf"contract_pair(_kernel)?(<{nb},|ILi{nb}E)|contract(_kernel)?(<{nb}, .*_Float16>|ILi{nb}E.*DF16_EE)"}.get(kernel)
     if pat is None:
         return None
-    import re
     hits = [v for k, v in summ["kernels"].items() if re.search(pat, k)]
     if not hits:
         return None
@@ -409,6 +411,7 @@ def _short_kernel_name(sym):
     'attn_bwd_dkv<32, 7>' (the event timer's name plus the template
     arguments, which tell head widths and lengths apart)."""
     s = sym.replace("(anonymous namespace)::", "").replace("void ", "").replace("bc2n::", "")
+    s = re.sub(r"\((?:\w+::)*\w+\)(?=\d)", "", s)  # an enum argument prints as a cast
     s = s.split("(")[0] if not s.startswith("_Z") else s
     base, _, targs = s.partition("<")
     base = base.split("::")[-1]
