@@ -424,6 +424,10 @@ kernel(Args a, Epi epi) {
 // (8.0 against 9.3 at 36864, 72 against 74 at 262144).  Triangle attention's LN
 // takes 48 where 64-row workgroups come to one round and a little, or to much
 // less than one (18.1 against 20.6 at 36864, 26.5 / 27.3 at 50176; 33 / 30 at 65536).
+// From 448 rows a CU it takes 96: the 128 KB of weight fragments a workgroup reads
+// from L2 serve half as many rows again (64 / 96 rows by events: 57.9 / 56.5 at
+// 102400, 64.6 / 63.4 at 123904, 85.5 / 83.2 at 173056, 124 / 115 at 262144, 191 /
+// 173 at 409600; with trimul's column outputs 125 / 152 at 262144).
 template <In IN, int C, int H, bool FAST, class Epi>
 void launch(hipStream_t st, const Args& a, const Epi& epi) {
   static_assert(H == 0 || H == 4, "bias heads 0 or 4");
@@ -459,6 +463,10 @@ void launch(hipStream_t st, const Args& a, const Epi& epi) {
     if constexpr (C == 128 && IN == In::LN && !Epi::kHasCol) {
       if (per_cu > 112 && per_cu < 224) {
         width(integral_constant<int, 3>());
+        return;
+      }
+      if (per_cu > 448) {
+        width(integral_constant<int, 6>());
         return;
       }
     }
