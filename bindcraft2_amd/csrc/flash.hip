@@ -46,6 +46,10 @@
 namespace bc2n {
 
 constexpr float NEG_LOGIT = -8192.0f;
+// The mask added to a score before its product (the forward beyond N = 256):
+// absorbs every score of finite binary16 operands (below 2^38), so a masked key
+// holds it whatever its content, where NEG_LOGIT plus the score would not.
+constexpr float MASKED_ADD = -1e30f;
 
 // Row stride (in h16) of the LDS token x head-width tiles.  gfx950's LDS
 // serves a wave's 8-byte transposed read in two 32-lane halves of 256 bytes
@@ -210,9 +214,9 @@ __device__ __forceinline__ RowHeadQb row_tile_order(int bid, int R, int H, int n
 // 124 / 205 so.  Two rows a workgroup, the bias shared in registers, leave three
 // waves a SIMD and are slower (71 / 169 / 222), and so are 5 to 7 waves (56 / 131
 // / 209): too few workgroups a CU.
-// A masked key's score is NEG_LOGIT plus its unmasked score: weight exactly 0
-// beside any live key.  In a fully masked row the bias factor `br` and q are 0,
-// so every key scores exactly NEG_LOGIT and the row attends uniformly.
+// A masked key's score is MASKED_ADD: weight exactly 0 beside any live key.  In a
+// fully masked row the bias factor `br` and q are 0, so every key scores exactly
+// that, the row attends uniformly and its lse is that of NEG_LOGIT scores.
 // Online softmax across chunks: the output accumulator and the row sum are
 // rescaled once per chunk.
 template <int D, int NKB, int CB>
@@ -227,7 +231,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
   constexpr int NCH = NFULL + (TAIL ? 1 : 0);
   const int H = a.H;
   h16* KV = reinterpret_cast<h16*>(smem_raw);            // [2][K, V][CN][LD]
-  float* Ma = reinterpret_cast<float*>(KV + 4 * CN * LD);  // [N] 0 / NEG_LOGIT
+  float* Ma = reinterpret_cast<float*>(KV + 4 * CN * LD);  // [N] 0 / MASKED_ADD
 
   constexpr int nqb = (N + QR - 1) / QR;
   const long G = (long)a.R * H * nqb;
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
   for (int k = tid; k < N; k += T) {
     const bool o = a.mask[r * a.mask_sr + k * a.mask_sk] != 0.f;
     on |= o;
-    Ma[k] = o ? 0.f : NEG_LOGIT;
+    Ma[k] = o ? 0.f : MASKED_ADD;
   }
 
   const int q0 = qb * QR + wave * 16 * QT;
@@ -392,7 +396,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
       *reinterpret_cast<h16x4*>(a.o + orow + d0) = ov;
       *reinterpret_cast<h16x4*>(a.og + orow + d0) = gov;
     }
-    if (g == 0) a.lse[((long)r * H + h) * N + q] = mx[t] + __log2f(lsum);
+    if (g == 0) a.lse[((long)r * H + h) * N + q] = (br != 0.f ? mx[t] : NEG_LOGIT) + __log2f(lsum);
   }
 }
 
