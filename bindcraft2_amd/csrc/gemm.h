@@ -571,6 +571,27 @@ __global__ __launch_bounds__(256) void gemm_few_kernel(GemmArgs g, int split, Ep
 // Slices at most (their partials share a workgroup's LDS: 36 KB for 16).
 constexpr int GEMM_FEW_MAX_SLICES = 16;
 
+// Whether a product of `split` slices is one for the few-tile launch.  Its tiles
+// read every fragment from memory for themselves, where a 128 x 128 tile serves
+// 128 rows from one, so it loses once there is enough of it: counted in 32-deep
+// steps of 16 x 32 tiles a CU.  us a launch, few-tile / 128 x 128 (the split one
+// with its reduction):
+//   unsplit, K <= 128 (any K: as many tiles): 28 steps 7.2 / 7.2, 32 7.5 / 6.9, 48 9.5 / 7.8
+//   2 or 3 slices: K = 256 64 steps 10.2 / 14.4, 72 12.6 / 14.4, 112 16.3 / 19.0, but the
+//     MSA row attention's backward, whose f32 operand each tile scales for itself, 9 us
+//     the slower there; K = 384 180 25 / 21; K = 512 192 25 / 17; K = 1024, a wave's whole
+//     chain, 96 16.7 / 16.0, 384 46 / 19
+//   4 and more: K = 1024 256 steps 14.7 / 21.8, 320 20.0 / 20.2, and in place 336
+//     20.8 / 18.8; K = 2048 128 13.9 / 24.7, 160 18.7 / 15.7, 384 24.6 / 19.4
+inline bool gemm_few_fits(const GemmArgs& g, int split) {
+  if (split > GEMM_FEW_MAX_SLICES) return false;
+  const long cus = device_cus(), k32 = g.K / 32;
+  const long tiles = (long)((g.M + 15) / 16) * ((g.N + 31) / 32);
+  if (split == 1) return tiles * std::min(k32, 4L) <= 28 * cus;
+  if (split < 4) return g.K <= 512 && tiles * k32 <= 80 * cus;
+  return tiles * k32 <= (g.K <= 1024 ? 288 : 128) * cus;
+}
+
 // Both operands K-contiguous, one batch entry, `split` slices of a multiple
 // of 32.  16-row tiles while they leave CUs to fill; the 32 x 64 tile, which
 // reads half the operand bytes a product, once 16 x 32 tiles exceed four a CU
@@ -688,7 +709,7 @@ void gemm(hipStream_t st, const GemmArgs& g, const Epi& epi, const char* name = 
         split = (int)std::min<long>((device_cus() + tiles - 1) / tiles, g.K / 64);
         while (split > 1 && g.K / 32 % split != 0) --split;
       }
-      if (ak && bk && split <= GEMM_FEW_MAX_SLICES) {
+      if (ak && bk && gemm_few_fits(g, split)) {
         gemm_few(st, g, split, epi, al);
         return;
       }
