@@ -192,11 +192,16 @@ __device__ __forceinline__ RowHeadQb row_tile_order(int bid, int R, int H, int n
 }
 
 // ------------------------------------------------------------------ forward
-// Workgroup = (row r, head h, 128 queries); 4 waves x 32 queries (two 16-query
+// Workgroup = (row r, head h, 128 queries); 4 waves x 32 queries (QT = 2 16-query
 // tiles); N = 32*NKB > 256.  Keys are processed in chunks of 32 CB staged in
 // one of two LDS buffers, the next chunk's K and V loaded into registers while
 // the current one computes; one barrier a chunk.  A lane keeps its two queries'
 // scores of the chunk (8 keys of every block each) in registers.
+//
+// Where there are few workgroups a launch is one wave's chain of waits: then 8
+// waves x 16 queries (QT = 1), 128 keys a chunk, and each chunk's bias is loaded
+// before the barrier in front of it (N = 320, one row 7.4 us a launch; loaded
+// after it 8.4, with 32 queries a wave 10.6).
 //
 // No one unit bounds it: at N = 512 the bias reads from L2 (1 GB a launch) take
 // 30 us of 206, K and V's 15, the exponentials 14 (variants without each), about
@@ -219,13 +224,13 @@ __device__ __forceinline__ RowHeadQb row_tile_order(int bid, int R, int H, int n
 // that, the row attends uniformly and its lse is that of NEG_LOGIT scores.
 // Online softmax across chunks: the output accumulator and the row sum are
 // rescaled once per chunk.
-template <int D, int NKB, int CB>
-__global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
+template <int D, int NKB, int CB, int QT, int QW>
+__global__ __launch_bounds__(64 * QW) void attn_fwd_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   constexpr int DT = D / 16;
   constexpr int LD = lds_ld<D>();
   constexpr int N = 32 * NKB;  // == a.N (dispatch)
-  constexpr int QT = 2, QW = 4, T = 64 * QW, QR = 16 * QT * QW;  // queries a workgroup
+  constexpr int T = 64 * QW, QR = 16 * QT * QW;  // threads, queries a workgroup
   constexpr int CN = 32 * CB;  // keys per chunk
   constexpr int NFULL = NKB / CB, TAIL = NKB % CB;
   constexpr int NCH = NFULL + (TAIL ? 1 : 0);
@@ -280,6 +285,17 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
 #pragma unroll
     for (int i = 0; i < DT; ++i) acc[t][i] = z4;
   }
+  h16x8 bb[CB][QT];
+  auto load_bias = [&](int c, auto nbc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kb = 0; kb < decltype(nbc)::value; ++kb)
+#pragma unroll
+      for (int t = 0; t < QT; ++t)
+        if (QT > 1 || c * CB + kb < NKB)
+          bb[kb][t] = ld8(bias_frag_block(a.bias, h, (qw >> 4) + t, c * CB + kb, N, lane));
+  };
+  const std::integral_constant<int, CB> whole{};
+  if (QT == 1) load_bias(0, whole);
   nkv.store(KV, KV + CN * LD, tid, min(CN, N));
   if (NCH > 1)
     nkv.load(Kg + (long)CN * a.ld, a.ld, Vg + (long)CN * a.ld, a.ld, tid, min(CN, N - CN));
@@ -291,12 +307,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
     const h16* Ks = KV + (c & 1) * 2 * CN * LD;
     const h16* Vs = Ks + CN * LD;
     if (active) {
-      h16x8 bb[NBC][QT];
-#pragma unroll
-      for (int kb = 0; kb < NBC; ++kb)
-#pragma unroll
-        for (int t = 0; t < QT; ++t)
-          bb[kb][t] = ld8(bias_frag_block(a.bias, h, (qw >> 4) + t, (k0 >> 5) + kb, N, lane));
+      if (QT > 1) load_bias(c, nbc);
       f32x4 sv[NBC][2][QT];
       float mc[QT];
 #pragma unroll
@@ -318,6 +329,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
             sv[kb][kh][t] = HFrag<D>::mma(kf, qf[t], cs);  // score + bias + mask
           }
         }
+      if (QT == 1 && c + 1 < NCH) load_bias(c + 1, whole);
 #pragma unroll
       for (int kb = 0; kb < NBC; ++kb)
 #pragma unroll
@@ -613,16 +625,17 @@ __global__ __launch_bounds__(256) void attn_gate_bwd_kernel(AttnBwdArgs b) {
 // MFMA starts from bias - lse (one v_fma_mix_f32 from the binary16 bias) plus
 // the mask, -inf at masked keys so p = dS = 0 there; dP's from -Dsum.  K, V,
 // mask and transposed K reads, 64 LDS cycles a 32-key block, serve two query
-// tiles.  N = 288 / 416 / 512: 51 / 135 / 198 us a
+// tiles; where there are few workgroups QT = 1, 64 queries a workgroup (N = 320, one
+// row 5.8 us a launch; 8.6 with two tiles).  N = 288 / 416 / 512: 51 / 135 / 198 us a
 // launch with 16 queries a wave and 256 keys a chunk, 43 / 113 / 178 so.
-template <int D, int NKB, int CB>
-__global__ __launch_bounds__(256) void attn_bwd_dq_kernel(AttnBwdArgs b) {
+template <int D, int NKB, int CB, int QT, int QW>
+__global__ __launch_bounds__(64 * QW) void attn_bwd_dq_kernel(AttnBwdArgs b) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   constexpr int DT = D / 16;
   constexpr int LD = lds_ld<D>();
   const AttnArgs& a = b.f;
   constexpr int N = 32 * NKB;  // == a.N (dispatch)
-  constexpr int QT = 2, QW = 4, T = 64 * QW, QR = 16 * QT * QW;  // queries a workgroup
+  constexpr int T = 64 * QW, QR = 16 * QT * QW;  // threads, queries a workgroup
   constexpr int CN = 32 * CB;  // keys per chunk
   constexpr int NFULL = NKB / CB, TAIL = NKB % CB;
   constexpr int NCH = NFULL + (TAIL ? 1 : 0);
@@ -1976,6 +1989,13 @@ static const char* timer_name(int kernel, const AttnArgs& a) {
 // keys per LDS chunk of the forward / dQ kernels, rows per chunk of dK/dV
 static int attn_chunk(int N) { return N < 256 ? N : 256; }
 
+// Beyond N = 256, whether `g` workgroups of 128 queries leave the chip so idle
+// that the 16-query forms are the faster: up to two a CU (the MSA's few rows).  us,
+// 16 / 32 queries a wave, forward and dQ, 8 heads: N = 448, 1 row (32 workgroups)
+// 9.1 / 13.0 and 6.4 / 10.4, 16 rows (512) 15.4 / 16.7 and 13.9 / 14.6, 24 rows
+// (768) 22.8 / 20.6 and 19.0 / 18.4; N = 288, 16 rows (384) 9.6 / 11.2 and 8.5 / 10.0.
+static bool attn_few(long g) { return g <= 2L * device_cus(); }
+
 static void attn_check(const AttnArgs& a) {
   if (a.D != 32 && a.D != 16) throw std::runtime_error("attention: head width must be 16 or 32");
   if (a.N <= 0 || a.N % 32 != 0) throw std::runtime_error("attention: N must be a positive multiple of 32");
@@ -2002,13 +2022,26 @@ static void attn_fwd_t(hipStream_t st, const AttnArgs& a) {
     return;
   }
   if (!a.bias) throw std::runtime_error("attention: the chunked forward needs the pair bias");
-  const dim3 grid(xcd_grid((long)a.R * a.H * ((a.N + 127) / 128)));
+  const long G = (long)a.R * a.H * ((a.N + 127) / 128);
   with_blocks(a.N / 32, [&](auto nb) {
-    constexpr int NB = decltype(nb)::value, CB = NB >= 15 ? 3 : 2;  // key blocks a chunk
-    if constexpr (NB > 8) {
+    constexpr int NB = decltype(nb)::value;
+    // key blocks a chunk, 16-query tiles a wave, waves
+    auto go = [&](auto cb, auto qt, auto qw) {
+      constexpr int CB = decltype(cb)::value, QT = decltype(qt)::value, QW = decltype(qw)::value;
       // two K/V buffers and the key mask
       const size_t lds = (size_t)4 * 32 * CB * lds_ld<D>() * 2 + (size_t)a.N * 4;
-      hipLaunchKernelGGL((attn_fwd_kernel<D, NB, CB>), grid, dim3(256), lds, st, a);
+      const long g = (long)a.R * a.H * ((a.N + 16 * QT * QW - 1) / (16 * QT * QW));
+      hipLaunchKernelGGL((attn_fwd_kernel<D, NB, CB, QT, QW>), dim3(xcd_grid(g)), dim3(64 * QW), lds, st, a);
+    };
+    using std::integral_constant;
+    if constexpr (NB > 8) {
+      if constexpr (D == 32) {
+        if (attn_few(G)) {
+          go(integral_constant<int, 4>(), integral_constant<int, 1>(), integral_constant<int, 8>());
+          return;
+        }
+      }
+      go(integral_constant<int, NB >= 15 ? 3 : 2>(), integral_constant<int, 2>(), integral_constant<int, 4>());
     }
   });
 }
@@ -2051,12 +2084,24 @@ static void attn_bwd_t(hipStream_t st, const AttnBwdArgs& b0) {
   } else {
     if (!a.bias) throw std::runtime_error("attention: the chunked dQ needs the pair bias");
     KTimed kt(timer_name(2, a), st);
-    const dim3 grid(xcd_grid((long)a.R * a.H * ((a.N + 127) / 128)));  // as the forward
+    const long G = (long)a.R * a.H * ((a.N + 127) / 128);
     with_blocks(a.N / 32, [&](auto nb) {
-      constexpr int NB = decltype(nb)::value, CB = 2;  // key blocks a chunk
-      if constexpr (NB > 8) {
+      constexpr int NB = decltype(nb)::value;
+      auto go = [&](auto cb, auto qt, auto qw) {
+        constexpr int CB = decltype(cb)::value, QT = decltype(qt)::value, QW = decltype(qw)::value;
         const size_t lds = (size_t)4 * 32 * CB * lds_ld<D>() * 2 + (size_t)a.N * 4;
-        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NB, CB>), grid, dim3(256), lds, st, b);
+        const long g = (long)a.R * a.H * ((a.N + 16 * QT * QW - 1) / (16 * QT * QW));
+        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NB, CB, QT, QW>), dim3(xcd_grid(g)), dim3(64 * QW), lds, st, b);
+      };
+      using std::integral_constant;
+      if constexpr (NB > 8) {
+        if constexpr (D == 32) {
+          if (attn_few(G)) {
+            go(integral_constant<int, 2>(), integral_constant<int, 1>(), integral_constant<int, 4>());
+            return;
+          }
+        }
+        go(integral_constant<int, 2>(), integral_constant<int, 2>(), integral_constant<int, 4>());
       }
     });
   }
