@@ -113,13 +113,15 @@ struct has_tile<E, std::void_t<typename E::Tile>> : std::true_type {};
 // WC waves side by side over the columns, 4 / WC row groups (WC = 2 where nout
 // is 64).  64-row tiles with a front of their own keep three waves a SIMD: at
 // four they spill (trimul's projections 48 registers: 50 us instead of 28 at
-// N = 224).
+// N = 224).  Four waves are the most the others are given, for the registers'
+// sake, but the centre norm's 32-row form is free to run at five, where its
+// workgroups at N = 192 are one round (16.6 -> 15.5 us, N = 224 21.1 -> 20.5).
 template <In IN, int RT>
 constexpr int min_waves() {
   return RT >= 3 && (IN == In::LN || IN == In::CM || IN == In::GATED) ? 3 : 4;
 }
 template <In IN, int C, int RT, int WC, int H, bool FAST, class Epi>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(min_waves<IN, RT>(), 4))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(min_waves<IN, RT>(), IN == In::CM ? 8 : 4))) void
 kernel(Args a, Epi epi) {
   constexpr int BM = 16 * RT, LDX = C + 8, KS = C / 32, TI = RT * WC / 4;
   constexpr int LPR = C / 8, RPP = 256 / LPR, PASS = BM / RPP;  // lanes a row, rows a pass
@@ -339,7 +341,11 @@ kernel(Args a, Epi epi) {
     for (int i = 0; i < TI; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto product = [&](auto cols_c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+      for (int ks = 0; ks < KS; ++ks) {
+        // With column outputs the rows of every K step read ahead spill: their
+        // second half waits for the first half's products (the 20 to 60 bytes of
+        // scratch cost a launch about 1 us, trimul's projections).
+        if (IN == In::LN && Epi::kHasCol && ks == KS / 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
           const h16x8 xf = ld8(xs + ((wr * TI + i) * 16 + l16) * LDX + ks * 32 + 8 * g);
@@ -348,6 +354,7 @@ kernel(Args a, Epi epi) {
             acc[i][jj] = decltype(cols_c)::value ? mfma16x16x32(xf, bf[ks][jj], acc[i][jj])
                                                  : mfma16x16x32(bf[ks][jj], xf, acc[i][jj]);
         }
+      }
       // unconditional (the last chunk reloads its own): a load under a branch
       // leaves the in-order memory counter unknown at the join
       if constexpr (!ONE) load_b(min(j + 1, nch - 1));
