@@ -37,11 +37,12 @@ struct TriAttnW {
   int C = 0, H = 0, D = 0;
   const float *ln_g = nullptr, *ln_b = nullptr, *w2d = nullptr;  // w2d [C][H]
   const float* bqkvg = nullptr;  // [4HD]: zeros for q,k,v; gating_b for g
-  const h16* wqkvg_t = nullptr; // [4HD][C]
   // C = 128 or 64, H = 4: wqkvg_t, wo_t and wo in proj_frags order, wqkvg in
-  // the backward's dX kernel's
+  // the backward's dX kernel's; null otherwise, and the matrices below null here
+  // (but wqkvg at C = 128)
   const h16 *wqkvg_frag = nullptr, *wo_frag = nullptr, *wo_bfrag = nullptr, *dx_frag = nullptr;
   const h16* wqkvg = nullptr;   // [C][4HD]
+  const h16* wqkvg_t = nullptr; // [4HD][C]
   const h16* wo_t = nullptr;    // [C][HD]
   const h16* wo = nullptr;      // [HD][C]
   const float* bo = nullptr;     // [C]
@@ -70,12 +71,13 @@ struct TriMulW {
   int C = 0, I = 0;
   const float *ln_g = nullptr, *ln_b = nullptr, *cn_g = nullptr, *cn_b = nullptr;
   const float *bp = nullptr, *bg = nullptr, *bgl = nullptr, *bo = nullptr;
-  const h16* wcat = nullptr;    // [C][4I+C]  (GEMM column order)
-  const h16* wcat_t = nullptr;  // [4I+C][C]
   // I = C = 128 or 64: wcat_t, wo_t and wo in proj_frags order, and both
-  // products of the backward tail in its own
+  // products of the backward tail in its own; null otherwise, and the matrices
+  // below null here
   const h16 *wcat_frag = nullptr, *wo_frag = nullptr, *wo_bfrag = nullptr;
   const h16 *tail_w1 = nullptr, *tail_w2 = nullptr;
+  const h16* wcat = nullptr;    // [C][4I+C]  (GEMM column order)
+  const h16* wcat_t = nullptr;  // [4I+C][C]
   const h16* wo = nullptr;      // [I][C]
   const h16* wo_t = nullptr;    // [C][I]
 };
@@ -95,7 +97,7 @@ struct TransW {
   const float *ln_g = nullptr, *ln_b = nullptr, *b1 = nullptr, *b2 = nullptr;
   const h16 *w1 = nullptr, *w1_t = nullptr, *w2 = nullptr, *w2_t = nullptr;
   // C = 128, F = 4 and C = 64, F = 2: both products' B operands in MFMA fragment order, per
-  // direction (forward W1^T / W2^T, backward W2 / W1)
+  // direction (forward W1^T / W2^T, backward W2 / W1), in place of those above
   const h16 *frag1_f = nullptr, *frag2_f = nullptr, *frag1_b = nullptr, *frag2_b = nullptr;
 };
 TransW transition_weights(WeightStore& ws, const std::string& prefix);

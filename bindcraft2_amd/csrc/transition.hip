@@ -405,11 +405,12 @@ TransW transition_weights(WeightStore& ws, const std::string& P) {
   w.b1 = ws.f32(P + "transition1/bias");
   w.b2 = ws.f32(P + "transition2/bias");
   const HostTensor& w2 = ws.host(P + "transition2/weights");  // [F*C, C]
-  w.w1 = ws.derived<h16>("trans.w1:" + P, [&] { return to_h16(w1.data); });
-  w.w1_t = ws.derived<h16>("trans.w1_t:" + P, [&] { return transpose_h16(w1.data.data(), C, H); });
-  w.w2 = ws.derived<h16>("trans.w2:" + P, [&] { return to_h16(w2.data); });
-  w.w2_t = ws.derived<h16>("trans.w2_t:" + P, [&] { return transpose_h16(w2.data.data(), H, C); });
-  if (tf::width(C, H)) {
+  if (!tf::width(C, H)) {  // the GEMMs' forms
+    w.w1 = ws.derived<h16>("trans.w1:" + P, [&] { return to_h16(w1.data); });
+    w.w1_t = ws.derived<h16>("trans.w1_t:" + P, [&] { return transpose_h16(w1.data.data(), C, H); });
+    w.w2 = ws.derived<h16>("trans.w2:" + P, [&] { return to_h16(w2.data); });
+    w.w2_t = ws.derived<h16>("trans.w2_t:" + P, [&] { return transpose_h16(w2.data.data(), H, C); });
+  } else {
     const float* a1 = w1.data.data();  // [C][H]
     const float* a2 = w2.data.data();  // [H][C]
     w.frag1_f = ws.derived<h16>("trans.frag1_f:" + P, [&] {

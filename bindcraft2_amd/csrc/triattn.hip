@@ -255,18 +255,29 @@ TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
     }
     return c;
   };
-  w.wqkvg = ws.derived<h16>("triattn.wqkvg:" + P, [&] { return to_h16(cat()); });
-  w.wqkvg_t = ws.derived<h16>("triattn.wqkvg_t:" + P, [&] {
-    std::vector<float> c = cat();
-    return transpose_h16(c.data(), C, 4 * HD);
-  });
   const bool rows = (C == 128 || C == 64) && w.H == 4;  // the row-tile kernels' widths
+  // the dX product's GEMM reads it at the row kernels' C = 128 too, at large M
+  if (!rows || C == 128) w.wqkvg = ws.derived<h16>("triattn.wqkvg:" + P, [&] { return to_h16(cat()); });
+  const HostTensor& ow = ws.host(P + "attention/output_w");  // [H,D,C]
   if (rows) {
     w.wqkvg_frag = ws.derived<h16>("triattn.wqkvg_frag:" + P, [&] {
       const std::vector<float> c = cat();  // [C][4HD]
       return proj_frags(4 * HD, C, 0, [&](int n, int k) { return c[(size_t)k * 4 * HD + n]; });
     });
     w.dx_frag = ws.derived<h16>("triattn.dx_frag:" + P, [&] { return dx_frags(cat(), C); });
+    w.wo_frag = ws.derived<h16>("triattn.wo_frag:" + P, [&] {
+      return proj_frags(C, HD, C, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
+    });
+    w.wo_bfrag = ws.derived<h16>("triattn.wo_bfrag:" + P, [&] {
+      return proj_frags(HD, C, 0, [&](int n, int k) { return ow.data[(size_t)n * C + k]; });
+    });
+  } else {  // the GEMMs' forms
+    w.wqkvg_t = ws.derived<h16>("triattn.wqkvg_t:" + P, [&] {
+      std::vector<float> c = cat();
+      return transpose_h16(c.data(), C, 4 * HD);
+    });
+    w.wo = ws.derived<h16>("triattn.wo:" + P, [&] { return to_h16(ow.data); });
+    w.wo_t = ws.derived<h16>("triattn.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), HD, C); });
   }
   w.bqkvg = ws.derived<float>("triattn.bqkvg:" + P, [&] {
     std::vector<float> b((size_t)4 * HD, 0.f);
@@ -274,18 +285,7 @@ TriAttnW triattn_weights(WeightStore& ws, const std::string& P) {
     for (int j = 0; j < HD; ++j) b[3 * HD + j] = gb.data[j];
     return b;
   });
-  const HostTensor& ow = ws.host(P + "attention/output_w");  // [H,D,C]
-  w.wo = ws.derived<h16>("triattn.wo:" + P, [&] { return to_h16(ow.data); });
-  w.wo_t = ws.derived<h16>("triattn.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), HD, C); });
   w.bo = ws.f32(P + "attention/output_b");
-  if (rows) {
-    w.wo_frag = ws.derived<h16>("triattn.wo_frag:" + P, [&] {
-      return proj_frags(C, HD, C, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
-    });
-    w.wo_bfrag = ws.derived<h16>("triattn.wo_bfrag:" + P, [&] {
-      return proj_frags(HD, C, 0, [&](int n, int k) { return ow.data[(size_t)n * C + k]; });
-    });
-  }
   return w;
 }
 

@@ -649,30 +649,28 @@ TriMulW trimul_weights(WeightStore& ws, const std::string& P) {
     }
     return c;
   };
-  w.wcat = ws.derived<h16>("trimul.wcat:" + P, [&] { return to_h16(cat()); });
-  w.wcat_t = ws.derived<h16>("trimul.wcat_t:" + P, [&] {
-    std::vector<float> c = cat();
-    return transpose_h16(c.data(), C, NC);
-  });
-  const bool rows = I == C && (C == 128 || C == 64);  // the row-tile kernels' widths
-  if (rows) {
+  const HostTensor& ow = ws.host(P + "output_projection/weights");  // [I, C]
+  if (I == C && (C == 128 || C == 64)) {  // the row-tile kernels' widths and forms
     w.wcat_frag = ws.derived<h16>("trimul.wcat_frag:" + P, [&] {
       const std::vector<float> c = cat();  // [C][NC]
       return proj_frags(NC, C, 4 * I, [&](int n, int k) { return c[(size_t)k * NC + n]; });
     });
     w.tail_w1 = ws.derived<h16>("trimul.tail_w1:" + P, [&] { return tail_frags1(cat(), C); });
     w.tail_w2 = ws.derived<h16>("trimul.tail_w2:" + P, [&] { return tail_frags2(cat(), C); });
-  }
-  const HostTensor& ow = ws.host(P + "output_projection/weights");  // [I, C]
-  w.wo = ws.derived<h16>("trimul.wo:" + P, [&] { return to_h16(ow.data); });
-  w.wo_t = ws.derived<h16>("trimul.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), I, C); });
-  if (rows) {
     w.wo_frag = ws.derived<h16>("trimul.wo_frag:" + P, [&] {
       return proj_frags(C, I, 0, [&](int n, int k) { return ow.data[(size_t)k * C + n]; });
     });
     w.wo_bfrag = ws.derived<h16>("trimul.wo_bfrag:" + P, [&] {
       return proj_frags(I, C, 0, [&](int n, int k) { return ow.data[(size_t)n * C + k]; });
     });
+  } else {  // the GEMMs'
+    w.wcat = ws.derived<h16>("trimul.wcat:" + P, [&] { return to_h16(cat()); });
+    w.wcat_t = ws.derived<h16>("trimul.wcat_t:" + P, [&] {
+      std::vector<float> c = cat();
+      return transpose_h16(c.data(), C, NC);
+    });
+    w.wo = ws.derived<h16>("trimul.wo:" + P, [&] { return to_h16(ow.data); });
+    w.wo_t = ws.derived<h16>("trimul.wo_t:" + P, [&] { return transpose_h16(ow.data.data(), I, C); });
   }
   return w;
 }
