@@ -302,7 +302,8 @@ static void triattn_check(const TriAttnW& w, int N) {
 }
 
 
-// The forward with its scratch (xn [M][C], og [M][HD], binary16) supplied.
+// The forward with its scratch (og [M][HD] and, without the row kernels' weights,
+// xn [M][C], binary16) supplied.
 static void triattn_fwd_with(hipStream_t st, const TriAttnW& w, bool per_column, int N,
                              const float* pair_in, const float* mask, const float* tbl,
                              float* pair_out, void* save, h16* xn, h16* og) {
@@ -372,8 +373,9 @@ void triattn_fwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   const long M = (long)N * N;
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
-  ar.reset(st, (size_t)M * C * 2 + (size_t)M * HD * 2 + 1024);
-  h16* xn = ar.take_n<h16>((size_t)M * C);
+  const size_t nxn = w.wqkvg_frag ? 0 : (size_t)M * C;  // the row kernel keeps xn on chip
+  ar.reset(st, nxn * 2 + (size_t)M * HD * 2 + 1024);
+  h16* xn = nxn ? ar.take_n<h16>(nxn) : nullptr;
   h16* og = ar.take_n<h16>((size_t)M * HD);
   triattn_fwd_with(st, w, per_column, N, pair_in, mask, tbl, pair_out, save, xn, og);
 }
@@ -440,19 +442,21 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   cs = module_scale_lazy(st, cs, dout, M * C);
   // the row kernel below reduces a scale still in partials; the GEMM does not
   const float* sc = w.wo_bfrag ? cs.sc : ct_scale_now(st, cs);
+  b.dbias_deferred = w.dx_frag != nullptr;  // the dX product's kernel adds the partials
+  const bool sum = nch == 1 || !b.dbias_deferred;  // the whole gradient: one partial, or the reduction's
   Sizer need;
   need.take<h16>((size_t)M * HD);           // dO
   need.take<float>((size_t)H * M);           // Dsum
   need.take<h16>((size_t)M * 4 * HD);       // dqkvg
   need.take<float>((size_t)nch * H * M);     // dbias partials
-  need.take<float>((size_t)H * M);           // dbias
+  if (sum) need.take<float>((size_t)H * M);  // dbias
   if (!w.dx_frag) need.take<float>((size_t)M * C);  // dxn
   ar.reset(st, need.off);
   b.dO = ar.take_n<h16>((size_t)M * HD);
   b.nDsum = ar.take_n<float>((size_t)H * M);
   b.dqkvg = ar.take_n<h16>((size_t)M * 4 * HD);
   b.dbias_part = ar.take_n<float>((size_t)nch * H * M);
-  b.dbias = ar.take_n<float>((size_t)H * M);
+  b.dbias = sum ? ar.take_n<float>((size_t)H * M) : nullptr;
   float* dxn = w.dx_frag ? nullptr : ar.take_n<float>((size_t)M * C);
 
   // d(og) = (tbl * dout) . Wo^T, the dropout scale applied as A is loaded;
@@ -490,7 +494,6 @@ void triattn_bwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
   a.o = sv.o; a.og = nullptr; a.ldo = HD;
   a.lse = sv.lse;
   b.scale = 1.f / std::sqrt((float)w.D);
-  b.dbias_deferred = w.dx_frag != nullptr;  // the dX product's kernel adds the partials
   attn_bwd(st, b);
 
   if (w.dx_frag && triattn_dx_fits(C, M)) {

@@ -731,9 +731,12 @@ void trimul_fwd(hipStream_t st, const TriMulW& w, bool outgoing, int N, const fl
   TriMulSave<Carver> sv(cv, N, C, I);
   Arena& ar = arena();
   std::lock_guard<std::recursive_mutex> lk(ar.lock());
-  ar.reset(st, (size_t)M * I * 2 + 1024);
   h16* xn = sv.xn;
-  h16* tn = ar.take_n<h16>((size_t)M * I);
+  h16* tn = nullptr;  // the row kernel keeps it on chip
+  if (!w.wo_frag) {
+    ar.reset(st, (size_t)M * I * 2 + 1024);
+    tn = ar.take_n<h16>((size_t)M * I);
+  }
   const EpiTrimulProj proj{sv.left, sv.right, sv.gout, w.bp, w.bg, w.bgl, mask, M, I, C};
   if (w.wcat_frag) {
     lnproj::Args la{};
