@@ -101,11 +101,12 @@ def kernel_model(name, n):
         "trimul.contract_bwd": (4 * c * n ** 3, m * 10 * c) if n <= 256 else
                                (2 * c * n ** 3, m * 6 * c),
         "triattn.gemm_qkvg": (gemm(c, 4 * c), m * (2 * c + 8 * c)),
-        # input LayerNorm + bias heads + q|k|v|g projection in one kernel:
-        # pair read, xn + statistics + bias + qkvg written
-        # input LayerNorm + the 4I + C projection columns in one kernel
+        # input LayerNorm + the 4I + C projection columns in one kernel: pair and
+        # mask read, xn, statistics, left, right and the output gate written
         "trimul.ln_proj": (gemm(c, 5 * c), m * (4 * c + 2 * c + 8 + 4 + 2 * 2 * c + 2 * c)),
-        "triattn.ln_qkvg": (gemm(c, 4 * c), m * (4 * c + 2 * c + 8 + 4 * h + 8 * c)),
+        # input LayerNorm + bias heads + q|k|v|g projection in one kernel: pair
+        # read, statistics, bias (binary16) and qkvg written; xn stays on chip
+        "triattn.ln_qkvg": (gemm(c, 4 * c), m * (4 * c + 8 + 2 * h + 8 * c)),
         "triattn.gemm_out": (gemm(c, c), m * (2 * c + 4 * c + 4 * c)),
         "triattn.gemm_dout": (gemm(c, c), m * (4 * c + 8 * c + 4 * h)),
         "triattn.gemm_dx": (gemm(4 * c, c), m * (8 * c + 4 * c)),
@@ -301,8 +302,8 @@ def traffic_of(kernel, n):
     # the triangle-attention launches are the head-width-32 instantiation (the
     # row-chunk forms for N <= 256); other timer names map to no one symbol
     nb = n // 32
-    syms = {"attn_fwd": [f"attn_fwd_rows<32, {nb}>", *(f"attn_fwd<32, {nb}, {cb}>" for cb in (2, 3))],
-            "attn_bwd_dq": [f"attn_bwd_dq_rows<32, {nb}>", f"attn_bwd_dq<32, {nb}, 2>"],
+    syms = {"attn_fwd": [f"attn_fwd_rows<32, {nb}>", *(f"attn_fwd<32, {nb}, {cb}, 2, 4>" for cb in (2, 3))],
+            "attn_bwd_dq": [f"attn_bwd_dq_rows<32, {nb}>", f"attn_bwd_dq<32, {nb}, 2, 2, 4>"],
             "attn_bwd_dkv": [f"attn_bwd_dkv_lds<{nb}>", f"attn_bwd_dkv_lds8<{nb}>",
                              f"attn_bwd_dkv<32, {nb}, {8 if nb > 8 else 4}, "
                              f"{8 if nb > 24 else 4 if nb > 8 else 2}>"],
