@@ -215,10 +215,12 @@ __device__ __forceinline__ RowHeadQb row_tile_order(int bid, int R, int H, int n
 //    the P V product itself (one more MFMA per block with an all-ones operand),
 //    summed over the same h16 probabilities the numerator uses.
 //  * 64 keys a chunk (113 registers: four waves a SIMD); 96 from N = 480.
-// N = 288 / 416 / 512: 54 / 140 / 218 us a launch with 16 queries a wave, 50 /
-// 124 / 205 so.  Two rows a workgroup, the bias shared in registers, leave three
-// waves a SIMD and are slower (71 / 169 / 222), and so are 5 to 7 waves (56 / 131
-// / 209): too few workgroups a CU.
+// In triangle attention's pass, N = 288 / 416 / 512: 63 / 160 / 242 us a launch with
+// 16 queries a wave and 128 keys a chunk, 56 / 146 / 223 so.  The launch repeated by
+// itself, its inputs in cache, 54 / 140 / 218 and 50 / 124 / 205; measured that way,
+// two rows a workgroup, the bias shared in registers, leave three waves a SIMD and
+// are slower (71 / 169 / 222), and so are 5 to 7 waves (56 / 131 / 209): too few
+// workgroups a CU.
 // A masked key's score is MASKED_ADD: weight exactly 0 beside any live key.  In a
 // fully masked row the bias factor `br` and q are 0, so every key scores exactly
 // that, the row attends uniformly and its lse is that of NEG_LOGIT scores.
@@ -626,8 +628,9 @@ __global__ __launch_bounds__(256) void attn_gate_bwd_kernel(AttnBwdArgs b) {
 // the mask, -inf at masked keys so p = dS = 0 there; dP's from -Dsum.  K, V,
 // mask and transposed K reads, 64 LDS cycles a 32-key block, serve two query
 // tiles; where there are few workgroups QT = 1, 64 queries a workgroup (N = 320, one
-// row 5.8 us a launch; 8.6 with two tiles).  N = 288 / 416 / 512: 51 / 135 / 198 us a
-// launch with 16 queries a wave and 256 keys a chunk, 43 / 113 / 178 so.
+// row 5.8 us a launch; 8.6 with two tiles).  In the pass, N = 288
+// / 416 / 512: 60 / 144 / 206 us a launch with 16 queries a wave and 256 keys a
+// chunk, 51 / 123 / 183 so.
 template <int D, int NKB, int CB, int QT, int QW>
 __global__ __launch_bounds__(64 * QW) void attn_bwd_dq_kernel(AttnBwdArgs b) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];

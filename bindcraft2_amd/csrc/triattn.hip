@@ -381,12 +381,13 @@ void triattn_fwd(hipStream_t st, const TriAttnW& w, bool per_column, int N,
 }
 
 // ------------------------------------------------- the allocation-free variant
-// Its scratch (xn and og of triattn_fwd_with) is this file-scope device
-// array: one copy per GPU, allocated with the code object, held until the
-// process ends.  Host code never passes `scratch` itself (its host-side name
-// is a stand-in, not a device address): the first call on each device looks
-// up the device address with hipGetSymbolAddress and keeps it per device.
-// Calls on one GPU share the array, so calls that overlap on one GPU race.
+// Its scratch (xn and og of triattn_fwd_with, xn's part counted in the limit
+// whether the path uses it or not) is this file-scope device array: one copy
+// per GPU, allocated with the code object, held until the process ends.  Host
+// code never passes `scratch` itself (its host-side name is a stand-in, not a
+// device address): the first call on each device looks up the device address
+// with hipGetSymbolAddress and keeps it per device.  Calls on one GPU share the
+// array, so calls that overlap on one GPU race.
 static __device__ __align__(256) unsigned char scratch[TRIATTN_NOALLOC_SCRATCH_BYTES];
 
 static void* scratch_ptr() {
